@@ -32,6 +32,7 @@ from __future__ import annotations
 import torch
 
 from . import _lib
+from .int8_gemm import _ROW_DTYPES as _QUANT_DTYPES
 
 
 def _bf16(t: torch.Tensor, what: str) -> torch.Tensor:
@@ -44,6 +45,13 @@ def _bf16(t: torch.Tensor, what: str) -> torch.Tensor:
     return t.contiguous()
 
 
+def _index_vector(indices):
+    """indices as a contiguous int64 vector: the tensor itself when it is one."""
+    if indices.dim() == 1 and indices.dtype == torch.int64 and indices.is_contiguous():
+        return indices
+    return indices.reshape(-1).contiguous().to(torch.int64)
+
+
 def _norm_args(source, norm, table, indices):
     source = _bf16(source, "source")
     _lib.check_device(source)
@@ -53,9 +61,7 @@ def _norm_args(source, norm, table, indices):
     _lib.same_device(source, **{"norm.weight": weight}, table=table, indices=indices)
     weight = _bf16(weight, "norm.weight")
     table = _bf16(table, "table")
-    indices = indices.reshape(-1).contiguous()
-    if indices.dtype != torch.int64:
-        indices = indices.to(torch.int64)
+    indices = _index_vector(indices)
     hidden = source.shape[-1]
     sequence = source.shape[-2] if source.dim() >= 2 else 1
     if weight.numel() != hidden:
@@ -67,10 +73,6 @@ def _norm_args(source, norm, table, indices):
     return source, weight, table, indices, hidden, sequence, width, table_rows
 
 
-_QUANT_DTYPES = {torch.bfloat16: _lib.DTYPE_BF16, torch.float16: _lib.DTYPE_F16,
-                 torch.float32: _lib.DTYPE_F32}
-
-
 def quantize_rows(value):
     """Per-row symmetric INT8 quantizer (model/kernels.py:19-24) for bf16,
     fp16 or fp32 rows (the Triton kernel loads any float row as fp32)."""
@@ -80,8 +82,8 @@ def quantize_rows(value):
         raise RuntimeError(f"value: dtype {value.dtype} is not supported by the HIP quantizer")
     value = value.contiguous()
     _lib.check_device(value)
-    output = torch.empty_like(value, dtype=torch.int8)
-    scales = torch.empty(rows, 1, device=value.device, dtype=torch.float32)
+    output = value.new_empty((rows, width), dtype=torch.int8)
+    scales = value.new_empty((rows, 1), dtype=torch.float32)
     if dtype == _lib.DTYPE_BF16:
         _lib.call("lr_quantize_rows", value.data_ptr(), rows, width, output.data_ptr(),
                   scales.data_ptr(), _lib.stream(value))
@@ -132,8 +134,8 @@ def _rms_adaln_quant_int8(source, norm, table, indices, shift_slot, scale_slot):
     source, weight, table, indices, hidden, sequence, width, table_rows = _norm_args(
         source, norm, table, indices)
     rows = source.numel() // hidden
-    output = torch.empty((rows, hidden), device=source.device, dtype=torch.int8)
-    scales = torch.empty((rows, 1), device=source.device, dtype=torch.float32)
+    output = source.new_empty((rows, hidden), dtype=torch.int8)
+    scales = source.new_empty((rows, 1), dtype=torch.float32)
     _lib.call("lr_rms_adaln_quant", source.data_ptr(), weight.data_ptr(), table.data_ptr(),
               indices.data_ptr(), output.data_ptr(), scales.data_ptr(), rows, sequence, hidden,
               table_rows, width, int(shift_slot), int(scale_slot), float(norm.eps),
@@ -152,8 +154,8 @@ def residual_rms_quant(source, update, norm, table, indices):
         raise ValueError("update must have the shape of source")
     rows = source.numel() // hidden
     residual = torch.empty_like(source)
-    quantized = torch.empty((rows, hidden), device=source.device, dtype=torch.int8)
-    scales = torch.empty((rows, 1), device=source.device, dtype=torch.float32)
+    quantized = source.new_empty((rows, hidden), dtype=torch.int8)
+    scales = source.new_empty((rows, 1), dtype=torch.float32)
     _lib.call("lr_residual_rms_quant", source.data_ptr(), update.data_ptr(), weight.data_ptr(),
               table.data_ptr(), indices.data_ptr(), residual.data_ptr(), quantized.data_ptr(),
               scales.data_ptr(), rows, sequence, hidden, table_rows, width, float(norm.eps),
@@ -170,9 +172,7 @@ def _gated_residual(residual, update, table, indices, gate_slot):
     if update.shape != residual.shape:
         raise ValueError("update must have the shape of residual")
     table = _bf16(table, "table")
-    indices = indices.reshape(-1).contiguous()
-    if indices.dtype != torch.int64:
-        indices = indices.to(torch.int64)
+    indices = _index_vector(indices)
     hidden = residual.shape[-1]
     sequence = residual.shape[-2] if residual.dim() >= 2 else 1
     if indices.numel() < sequence:

@@ -67,6 +67,13 @@ extern "C" {
 #define LR_TILE_256x256_PERSISTENT 13 /* 256x256 on a persistent grid (one workgroup per CU looping
                                         over the tiles, each tile's last k-steps loading the next
                                         tile's first ones); replaces model/int8_tma.py:12-41 */
+/* Tiles between the large and the small-M ones: 8 waves on a 2x4 grid. */
+#define LR_TILE_224x256 14
+#define LR_TILE_160x256 15
+#define LR_TILE_192x128 16
+#define LR_TILE_128x192 17
+#define LR_TILE_96x128 18
+#define LR_TILE_LAST LR_TILE_96x128
 
 /* Library version; bumped whenever a signature below changes. */
 int lr_abi_version(void);

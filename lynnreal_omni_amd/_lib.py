@@ -27,7 +27,8 @@ EPI_BF16, EPI_GELU_TANH, EPI_GATED_RESIDUAL, EPI_RAW_INT32 = 0, 1, 2, 3
 DTYPE_BF16, DTYPE_F16, DTYPE_F32 = 0, 1, 2
 (TILE_AUTO, TILE_256x256, TILE_256x128, TILE_128x256, TILE_128x128, TILE_64x128, TILE_GENERIC,
  TILE_256x256_W4x2, TILE_256x192, TILE_256x80, TILE_64x80, TILE_128x160, TILE_192x256,
- TILE_256x256_PERSISTENT) = range(14)
+ TILE_256x256_PERSISTENT, TILE_224x256, TILE_160x256, TILE_192x128, TILE_128x192,
+ TILE_96x128) = range(19)
 ABI_VERSION = 1
 
 _P = ctypes.c_void_p
@@ -201,6 +202,11 @@ def workspace(t: torch.Tensor, nbytes: int) -> tuple[int | None, int]:
     the work already queued there."""
     if nbytes <= 0:
         return None, 0
+    if torch.cuda.is_current_stream_capturing():
+        # Memory of the graph being captured: a kept buffer could be outgrown
+        # and freed under the graph, or shared with another graph's replay.
+        buf = torch.empty(nbytes, dtype=torch.uint8, device=t.device)
+        return buf.data_ptr(), nbytes
     key = (t.get_device(), stream(t))
     buf = _workspaces.pop(key, None)
     if buf is None or buf.numel() < nbytes:

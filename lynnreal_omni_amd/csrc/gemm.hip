@@ -23,6 +23,7 @@
 //    tiles and its 4 MB L2 holds the A and W panels its CUs share.
 // Generic kernel: any W strides / K, LDS-tiled int32 dot products (slow path
 // used only when the fast kernel cannot run).
+#include <cmath>
 #include <mutex>
 
 #include "lr_device.h"
@@ -72,13 +73,13 @@
 #ifndef GEMM_SKINNY128_NB
 #define GEMM_SKINNY128_NB 4
 #endif
-// Staging rows whose residual and gate chunks the gated epilogue loads
-// before using any of them, where it divides the wave's rows of chunks (else
-// 4). Chain timings: 6 took FFN-down's 192x256 tiles (12 rows) from 900 to
+// Staging rows whose residual and gate chunks the gated epilogue loads before
+// using any of them: the largest divisor of the wave's rows of chunks up to
+// this. Chain timings: 6 took FFN-down's 192x256 tiles (12 rows) from 900 to
 // 896-897 us; 8 spills registers in the 256x256 tile (out-proj 281 -> 342 us)
 // and 12 in the 192x256 one (900 -> 1416 us).
 #ifndef GEMM_GATED_BATCH
-#define GEMM_GATED_BATCH 6
+#define GEMM_GATED_BATCH 7
 #endif
 // Rows of tiles per raster group of the XCD-aware tile order.
 #ifndef GEMM_GROUP_M
@@ -247,6 +248,13 @@ __device__ __forceinline__ void store_tile(const GemmArgs& p, const v4i (&acc)[F
   }
 }
 
+// The largest divisor of n that is at most `most`.
+constexpr int divisor_up_to(int n, int most) {
+  int d = n < most ? n : most;
+  while (n % d != 0) --d;
+  return d;
+}
+
 // Whole-line output stores, non-temporal: the output is not read again by
 // this kernel, and streaming it keeps the L2 for the operand panels (FFN-up
 // 1135 -> 1107 us, the other projections 1-2% faster).
@@ -318,8 +326,8 @@ __device__ __forceinline__ void store_tile_staged(const GemmArgs& p, const v4i (
   constexpr bool kWhole = WM * CPR % 64 == 0;   // else the last pass is partial
   static_assert(WN % 8 == 0, "staging tile shape");
   const bool seq_covers = p.sequence >= p.m;
-  if constexpr (EPI == EPI_GATED && WM <= 128 && kWhole && ITERS % 4 == 0) {
-    // x + bf16(gate * y): the residual and gate chunks of 4 staging rows are
+  if constexpr (EPI == EPI_GATED && WM <= 128 && kWhole && divisor_up_to(ITERS, GEMM_GATED_BATCH) >= 3) {
+    // x + bf16(gate * y): the residual and gate chunks of BATCH staging rows are
     // loaded before any of them is used, from clamped (always valid)
     // addresses, so the loads overlap instead of each waiting in turn (a load
     // under a branch, or after a store the compiler cannot prove disjoint,
@@ -334,7 +342,7 @@ __device__ __forceinline__ void store_tile_staged(const GemmArgs& p, const v4i (
     };
     const int tr_lane = table_row_of(lane);
     const int tr_lane_hi = WM > 64 ? table_row_of(64 + lane) : 0;
-    constexpr int BATCH = ITERS % GEMM_GATED_BATCH == 0 ? GEMM_GATED_BATCH : 4;
+    constexpr int BATCH = divisor_up_to(ITERS, GEMM_GATED_BATCH);
 #pragma unroll 1
     for (int s0 = 0; s0 < ITERS; s0 += BATCH) {
       uint4 xv[BATCH], gv[BATCH], v[BATCH];
@@ -612,11 +620,11 @@ __global__ __launch_bounds__(64 * WAVES_M * WAVES_N) void gemm_fast(GemmArgs p) 
     //
     // A slot of k-step k is free once group 1 has read it (its lgkmcnt(0)
     // before the barrier that ends phase 2k + 1). Group 0 refills the A ring
-    // (3 slots): A(k + 2) in its memory phase of k-step k, into the slot of
-    // k-step k - 1, and waits for A(k + 1) at the end of its compute phase of
-    // k-step k. Group 1 refills the W ring (2 slots) with W(k + 2), into the
-    // slot of k-step k, and waits for W(k + 1) before the barrier that ends its
-    // memory phase. Both waits land just before the barrier that ends phase
+    // (NA slots): A(k + NA - 1) in its memory phase of k-step k, into the slot
+    // of k-step k - 1, and waits for A(k + 1) at the end of its compute phase
+    // of k-step k. Group 1 refills the W ring (NB slots) with W(k + NB), into
+    // the slot of k-step k, and waits for W(k + 1) before the barrier that ends
+    // its memory phase. Both waits land just before the barrier that ends phase
     // 2k + 1, which publishes k-step k + 1 for group 0's read in phase 2k + 2.
     // A wave's DMAs write the q-th quarter of the tile's W rows (q = wave % 4).
     // With four waves across N (wn = q) no other wave of group 1 reads those
@@ -626,7 +634,7 @@ __global__ __launch_bounds__(64 * WAVES_M * WAVES_N) void gemm_fast(GemmArgs p) 
     // per-wave lgkmcnt does not cover other waves): the refill then waits for
     // the barrier that ends phase 2k + 1 and goes out at the start of group
     // 1's compute phase.
-    static_assert(NWAVES == 8 && NA == 3 && NB == 2 && KALIGNED, "ping-pong layout");
+    static_assert(NWAVES == 8 && NA >= 2 && NB >= 2 && KALIGNED, "ping-pong layout");
     constexpr int PA = BM / 8 / 4, PB = BN / 8 / 4;  // 1 KB DMAs per wave per k-step
     static_assert(PA * 32 == BM && PB * 32 == BN && PA <= 15 && PB <= 15, "ping-pong DMA split");
     const int grp = wave >> 2, q = wave & 3;
@@ -649,10 +657,13 @@ __global__ __launch_bounds__(64 * WAVES_M * WAVES_N) void gemm_fast(GemmArgs p) 
       for (int j = 0; j < PB; ++j)
         dma16s(rb, b_ring + (kt % NB) * B_BYTES + (q * PB + j) * 1024, pb_off[j], soff);
     };
-    constexpr int kWaitA = 0x70 | 0xf00 | PA;  // vmcnt(PA): all but the newest k-step landed
-    constexpr int kWaitB = 0x70 | 0xf00 | PB;
+    // All but the newest NA - 2 (A) or NB - 1 (W) k-steps landed.
+    constexpr int kVmA = (NA - 2) * PA, kVmB = (NB - 1) * PB, kVmB2 = (NB - 2) * PB;
+    static_assert(kVmA <= 63 && kVmB <= 63, "vmcnt range");
+    constexpr int kWaitA = 0x70 | 0xf00 | (kVmA & 0xf) | ((kVmA >> 4) << 14);
+    constexpr int kWaitB = 0x70 | 0xf00 | (kVmB & 0xf) | ((kVmB >> 4) << 14);
     constexpr int kWaitLds = 0xc07f;           // lgkmcnt(0)
-    constexpr int kWaitLdsVm0 = 0x70;          // vmcnt(0) lgkmcnt(0)
+    constexpr int kWaitLdsB2 = 0x70 | (kVmB2 & 0xf) | ((kVmB2 >> 4) << 14);  // and lgkmcnt(0)
     constexpr bool kOwnW = WAVES_N == 4;       // wn == wave % 4 for every wave
     v4i a0[FM], w0[FN], a1[FM], w1[FN];
     auto read_all = [&](int kt) {
@@ -688,13 +699,13 @@ __global__ __launch_bounds__(64 * WAVES_M * WAVES_N) void gemm_fast(GemmArgs p) 
       __builtin_amdgcn_sched_barrier(0);
     };
     if (grp == 0) {
-      pdma_a(0);
-      pdma_a(1);
+#pragma unroll
+      for (int t = 0; t < NA - 1; ++t) pdma_a(t);
       __builtin_amdgcn_s_waitcnt(kWaitA);
       barrier();
       for (int kt = 0; kt < KT; ++kt) {
         read_all(kt);  // phase 2kt
-        pdma_a(kt + 2);
+        pdma_a(kt + NA - 1);
         __builtin_amdgcn_s_waitcnt(kWaitLds);
         barrier();
         compute();  // phase 2kt + 1
@@ -704,8 +715,8 @@ __global__ __launch_bounds__(64 * WAVES_M * WAVES_N) void gemm_fast(GemmArgs p) 
       }
       barrier();  // phase 2KT: group 1 computes the last k-step
     } else {
-      pdma_b(0);
-      pdma_b(1);
+#pragma unroll
+      for (int t = 0; t < NB; ++t) pdma_b(t);
       __builtin_amdgcn_s_waitcnt(kWaitB);
       barrier();
       barrier();  // phase 0: group 0 reads k-step 0
@@ -714,17 +725,17 @@ __global__ __launch_bounds__(64 * WAVES_M * WAVES_N) void gemm_fast(GemmArgs p) 
         if constexpr (kOwnW) {
           // This wave alone in its group reads the W rows it refills.
           __builtin_amdgcn_s_waitcnt(kWaitLds);
-          pdma_b(kt + 2);
+          pdma_b(kt + NB);
           __builtin_amdgcn_s_waitcnt(kWaitB);  // W(kt + 1) landed
           barrier();
         } else {
           // Other waves of this group may still be reading the rows this
           // wave's DMAs would overwrite: refill after the barrier, by which
-          // every wave has read W(kt). W(kt + 1), issued one phase ago, is
-          // the only load in flight.
-          __builtin_amdgcn_s_waitcnt(kWaitLdsVm0);
+          // every wave has read W(kt). The loads in flight at the wait are
+          // W(kt + 1) .. W(kt + NB - 1); the first has landed after it.
+          __builtin_amdgcn_s_waitcnt(kWaitLdsB2);
           barrier();
-          pdma_b(kt + 2);
+          pdma_b(kt + NB);
         }
         compute();  // phase 2kt + 2
         barrier();
@@ -1297,19 +1308,24 @@ struct FastCfg {
   int bm, bn;
 };
 
+// RAGGED = false: the tile has no kernel for K % 128 != 0; such calls run the
+// 128x128 tile (the same outputs), which the automatic choice never needs.
 template <int BM, int BN, int WAVES_M, int WAVES_N, int EPI, bool BIAS, int NA = GEMM_RING_A,
-          int NB = GEMM_RING_B>
+          int NB = GEMM_RING_B, bool RAGGED = true>
 void launch_fast_cfg(GemmArgs& p, hipStream_t st) {
   p.tiles_m = (int)((p.m + BM - 1) / BM);
   p.tiles_n = (int)((p.n + BN - 1) / BN);
   const unsigned grid = (unsigned)(p.tiles_m * p.tiles_n * p.splits);
-  constexpr bool kPingPong = GEMM_PINGPONG && WAVES_M * WAVES_N == 8 && NA == 3 && NB == 2;
-  if (p.k % 128 == 0)
+  constexpr bool kPingPong = GEMM_PINGPONG && WAVES_M * WAVES_N == 8;
+  if (p.k % 128 == 0) {
     hipLaunchKernelGGL((gemm_fast<BM, BN, WAVES_M, WAVES_N, EPI, BIAS, NA, NB, true, kPingPong>),
                        dim3(grid), dim3(64 * WAVES_M * WAVES_N), 0, st, p);
-  else
+  } else if constexpr (RAGGED) {
     hipLaunchKernelGGL((gemm_fast<BM, BN, WAVES_M, WAVES_N, EPI, BIAS, NA, NB, false, false>),
                        dim3(grid), dim3(64 * WAVES_M * WAVES_N), 0, st, p);
+  } else {
+    launch_fast_cfg<128, 128, 2, 2, EPI, BIAS>(p, st);
+  }
 }
 
 // The persistent 256x256 block, streamed (K % 128 == 0 and K >= 256, else one
@@ -1349,9 +1365,13 @@ void launch_fast(int tile, GemmArgs& p, hipStream_t st) {
     // 8 waves of 64x96: 192-column tiles fill the CUs where 256-column ones leave a
     // partial wave (N = 5120 at M = 2048: 216 tiles instead of 160).
     case LR_TILE_256x192: launch_fast_cfg<256, 192, 4, 2, EPI, BIAS>(p, st); break;
-    // 4 waves of 128x64 / 64x128; two 48 KB k-steps.
-    case LR_TILE_256x128: launch_fast_cfg<256, 128, 2, 2, EPI, BIAS>(p, st); break;
-    case LR_TILE_128x256: launch_fast_cfg<128, 256, 2, 2, EPI, BIAS>(p, st); break;
+    case LR_TILE_256x128: launch_fast_cfg<256, 128, 2, 4, EPI, BIAS, 3, 2, false>(p, st); break;
+    case LR_TILE_128x256: launch_fast_cfg<128, 256, 2, 4, EPI, BIAS, 3, 2, false>(p, st); break;
+    case LR_TILE_224x256: launch_fast_cfg<224, 256, 2, 4, EPI, BIAS, 3, 2, false>(p, st); break;
+    case LR_TILE_160x256: launch_fast_cfg<160, 256, 2, 4, EPI, BIAS, 3, 2, false>(p, st); break;
+    case LR_TILE_192x128: launch_fast_cfg<192, 128, 2, 4, EPI, BIAS, 3, 3, false>(p, st); break;
+    case LR_TILE_128x192: launch_fast_cfg<128, 192, 2, 4, EPI, BIAS, 3, 3, false>(p, st); break;
+    case LR_TILE_96x128: launch_fast_cfg<96, 128, 2, 4, EPI, BIAS, 4, 4, false>(p, st); break;
     // 4 waves of 64x64; 80 KB of rings: 2 blocks per CU.
     case LR_TILE_128x128: launch_fast_cfg<128, 128, 2, 2, EPI, BIAS>(p, st); break;
     // 4 waves of 64x32 (24 KB k-steps), both operands GEMM_DEPTH_SMALL - 1
@@ -1421,38 +1441,102 @@ void dispatch_bias(bool generic, int tile, bool bias, GemmArgs& p, hipStream_t s
   }
 }
 
-int tile_rows(int tile) {
+struct TileShape {
+  int rows, cols;
+};
+
+TileShape tile_shape(int tile) {
   switch (tile) {
-    case LR_TILE_256x256: case LR_TILE_256x256_W4x2: case LR_TILE_256x128: case LR_TILE_256x192:
-    case LR_TILE_256x256_PERSISTENT:
-      return 256;
-    case LR_TILE_256x80: return 256;
-    case LR_TILE_192x256: return 192;
-    case LR_TILE_128x256: case LR_TILE_128x128: case LR_TILE_128x160: return 128;
-    default: return 64;
+    case LR_TILE_256x256: case LR_TILE_256x256_W4x2: case LR_TILE_256x256_PERSISTENT: return {256, 256};
+    case LR_TILE_256x192: return {256, 192};
+    case LR_TILE_256x128: return {256, 128};
+    case LR_TILE_256x80: return {256, 80};
+    case LR_TILE_224x256: return {224, 256};
+    case LR_TILE_192x256: return {192, 256};
+    case LR_TILE_192x128: return {192, 128};
+    case LR_TILE_160x256: return {160, 256};
+    case LR_TILE_128x256: return {128, 256};
+    case LR_TILE_128x192: return {128, 192};
+    case LR_TILE_128x160: return {128, 160};
+    case LR_TILE_128x128: return {128, 128};
+    case LR_TILE_96x128: return {96, 128};
+    case LR_TILE_64x80: return {64, 80};
+    default: return {64, 128};
   }
 }
-int tile_cols(int tile) {
-  switch (tile) {
-    case LR_TILE_256x256: case LR_TILE_256x256_W4x2: case LR_TILE_128x256: case LR_TILE_192x256:
-    case LR_TILE_256x256_PERSISTENT:
-      return 256;
-    case LR_TILE_256x192: return 192;
-    case LR_TILE_256x80: case LR_TILE_64x80: return 80;
-    case LR_TILE_128x160: return 160;
-    default: return 128;
-  }
+int tile_rows(int tile) { return tile_shape(tile).rows; }
+int tile_cols(int tile) { return tile_shape(tile).cols; }
+
+// ---------------------------------------------------- automatic schedule ----
+// The tile and the K split of a shape, by a model of the kernel's time (us) on
+// weights that come from HBM (a block's weights, read once per forward; a
+// loop over one weight runs from the 256 MB cache and is faster everywhere).
+//
+// A CU takes its operands at about 40-60 GB/s while they miss L2, whatever the
+// ring depth: loads return in order, so each waits behind the slowest. A
+// k-step of a BM x BN tile therefore costs c0 + c1 * (rows + cols) for its bytes
+// (rows past M are not read), together with cm * BM * BN for its MFMAs; a
+// tile adds f0 + f1 * BM * BN for its prologue and epilogue. Tiles run in waves
+// of one per CU; the last wave costs at least 0.9 of a full one, since its
+// tiles are as long, only with more bandwidth and clock. The weights' HBM time
+// (N * K at 5.5 TB/s) is a floor. S slices of K shorten the loops and fill
+// idle CUs, and cost a second launch and the write and read of S int32 partial
+// outputs (9 TB/s: they stay in the 256 MB cache).
+//
+// Fitted (log least squares, 6% rms over 5600 points) to graph-replayed times
+// with rotating weights: 12 tiles, up to 8 slices, M = 1 to 16385 on the eight
+// projections of the Flash model and of the 5120-wide block, bf16 and gated
+// epilogues. Over those 320 shapes its choice is within 1.1% of the fastest
+// (geometric mean), and 9% faster than the rules before it, which knew
+// neither the tiles marked * nor splits below K = 16384. Examples, before ->
+// now: M = 32, N = 5376, K = 7168 20.7 -> 15.1 us (64x80 in 3 slices);
+// M = 256, N = 5376, K = 14336 54.6 -> 36.3 us (128x192* in 4); M = 878, same N, K
+// 104 -> 78 us (128x160); M = 1500, N = 5120, K = 5120 47 -> 41 us (128x256*);
+// M = 10240, N = 5120, K = 20480 886 -> 804 us (224x256*).
+struct AutoTile {
+  int id, rows, cols;
+  double factor;  // against the model: 64x128 and 128x160 run one wave per SIMD
+};
+constexpr AutoTile kAutoTiles[] = {
+    {LR_TILE_256x256, 256, 256, 1.0},    {LR_TILE_224x256, 224, 256, 1.0},
+    {LR_TILE_192x256, 192, 256, 0.96},   {LR_TILE_160x256, 160, 256, 1.0},
+    {LR_TILE_256x128, 256, 128, 1.0},   {LR_TILE_128x256, 128, 256, 1.0},
+    {LR_TILE_192x128, 192, 128, 0.97},  {LR_TILE_128x192, 128, 192, 1.0},
+    {LR_TILE_128x160, 128, 160, 1.03},   {LR_TILE_96x128, 96, 128, 1.0},
+    {LR_TILE_64x128, 64, 128, 1.05},     {LR_TILE_64x80, 64, 80, 0.96},
+};
+// Automatic splits stay below this many slice bytes and slices: more never
+// measured faster by more than 7%, and callers hold the workspace.
+constexpr int64_t kAutoSliceBytes = 22LL << 20;
+constexpr int kAutoSlices = 8;
+
+double model_us(const AutoTile& t, int64_t m, int64_t n, int64_t k, int splits, int64_t cus) {
+  const int64_t tiles = ((m + t.rows - 1) / t.rows) * ((n + t.cols - 1) / t.cols) * splits;
+  const int64_t steps = ((k + 127) / 128 + splits - 1) / splits;
+  const int64_t full = tiles / cus, rest = tiles % cus;
+  const double waves = (double)full + (rest ? 0.9 + 0.1 * (double)rest / (double)cus : 0.0);
+  const double outputs = t.rows * t.cols * 1e-3;
+  const double bytes = 0.0624 + 0.00163 * (double)((m < t.rows ? m : t.rows) + t.cols);
+  const double mfma = 0.01425 * outputs;
+  const double loop = waves * t.factor *
+                      (2.7 + 0.054 * outputs + std::sqrt(bytes * bytes + mfma * mfma) * (double)steps);
+  const double weights = (double)n * (double)k * 1e-6 / 5.5;
+  double us = 4.2 + std::cbrt(loop * loop * loop + weights * weights * weights);
+  if (splits > 1) us += 2.6 + (double)splits * (double)m * (double)n * 8e-6 / 9.0;
+  return us;
 }
 
-// Shape heuristic from measured sweeps on MI355X (256 CUs, K = 5120 and
-// 20480, M from 64 to 12288, N from 5120 to 20480). A launch takes as many
+// K % 128 != 0 (the mid-step loop of gemm_fast; the tiles of the model above
+// that exist for it lose up to 22% to these rules, which also take 128x128 and
+// 256x192): shape heuristic from measured sweeps (256 CUs, K = 5120 and 20480,
+// M from 64 to 12288, N from 5120 to 20480). A launch takes as many
 // waves of tiles as its tile count fills the resident blocks of the device's
 // CUs (one 256x256, 192x256, 256x192 or 64x128 block per CU, two 128x128
 // blocks; a partitioned GPU has fewer CUs per device); each wave
 // costs a weight per tile (below), and the fewest weighted waves win, ties to
 // the larger tile. Past that, 256x256 and 192x256 are compared by a per-tile
 // time in K (long K favours 192x256 when it fills the waves better).
-int auto_tile(int64_t m, int64_t n, int64_t k) {
+int ragged_tile(int64_t m, int64_t n, int64_t k) {
   const int64_t cus = compute_units();
   auto tiles = [&](int t) { return ((m + tile_rows(t) - 1) / tile_rows(t)) * ((n + tile_cols(t) - 1) / tile_cols(t)); };
   // A few hundred rows (graph-replay timings at K = 5120): 64x80 when its
@@ -1496,22 +1580,6 @@ int auto_tile(int64_t m, int64_t n, int64_t k) {
   return c128 <= c64 ? LR_TILE_128x128 : LR_TILE_64x128;
 }
 
-// Split-K for a few hundred rows at long K, on 128x160 tiles: as many slices
-// as keep the workgroups within one wave of the device's CUs, at most 4 (1 =
-// no split).
-// Graph-replayed at M = 256, N = 5120, K = 20480 (bf16 + bias): 35.6 us for
-// 128x160 in 4 slices against 41.8 us unsplit on the shape's own tile. At
-// K = 5120 every split measured slower than the unsplit small-M tiles (the
-// partial slices' write and re-read, and the second launch, cost more than
-// the shorter k-loops save).
-int auto_splits(int64_t m, int64_t n, int64_t k) {
-  if (m > 256 || k < 16384 || k % 128 != 0 || n % 4 != 0) return 1;
-  const int64_t tiles = ((m + 127) / 128) * ((n + 159) / 160);
-  int64_t s = compute_units() / tiles;
-  if (s > 4) s = 4;
-  return s > 1 ? (int)s : 1;
-}
-
 }  // namespace
 }  // namespace lr
 
@@ -1533,29 +1601,73 @@ struct Plan {
   int splits;
 };
 
-// The fast-path schedule: the tile (LR_TILE_AUTO: by shape and epilogue) and
-// the split-K factor (splits 0: by shape when a workspace is allowed, else 1).
-// Where the shape takes 256x256 tiles over at least two waves of the chip and
-// the epilogue is bf16 or GELU, the persistent grid with streamed tiles runs
-// 1-2% faster than one tile per workgroup (QKV 12288x15360x5120: 660 against
-// 672 us, FFN-up 894 against 902-914 us, the Flash model's QKV and out-proj
-// shapes at full M likewise; same box). Its pass-staged gated epilogue is
-// slower (out-proj 286 against 265 us), so the gated and raw epilogues keep
-// one tile per workgroup.
-Plan plan(int64_t m, int64_t n, int64_t k, int tile, int splits, bool workspace, int epilogue) {
-  Plan pl{tile == LR_TILE_AUTO ? auto_tile(m, n, k) : tile, splits > 0 ? splits : 1};
-  if (splits == 0 && workspace && tile == LR_TILE_AUTO) {
-    const int s = auto_splits(m, n, k);
-    if (s > 1) pl = Plan{LR_TILE_128x160, s};
+int64_t split_workspace(int64_t m, int64_t n, int splits) { return splits > 1 ? splits * m * n * 4 : 0; }
+
+// The fastest (tile, splits) by the model, K % 128 == 0. splits 0: up to the workspace's
+// bytes; else that many. `streamed`: the epilogue can take the persistent grid
+// where 256x256 tiles make two waves of the chip or more.
+Plan search(int64_t m, int64_t n, int64_t k, int splits, int64_t workspace_bytes, bool streamed) {
+  const int64_t cus = compute_units();
+  const int64_t steps = (k + 127) / 128;
+  const int64_t budget = workspace_bytes < kAutoSliceBytes ? workspace_bytes : kAutoSliceBytes;
+  Plan best{LR_TILE_256x256, splits > 0 ? splits : 1};
+  double best_us = 0.0;
+  for (const AutoTile& t : kAutoTiles) {
+    const int64_t tiles = ((m + t.rows - 1) / t.rows) * ((n + t.cols - 1) / t.cols);
+    int last = splits > 0 ? splits : 1;
+    if (splits == 0 && n % 4 == 0) {
+      // Slices of at least 4 k-steps that make at most about one wave.
+      while (last < kAutoSlices && 4 * (last + 1) <= steps && tiles * last < cus &&
+             split_workspace(m, n, last + 1) <= budget)
+        ++last;
+    }
+    for (int s = splits > 0 ? splits : 1; s <= last; ++s) {
+      double us = model_us(t, m, n, k, s, cus);
+      // The streamed grid is 1-2% faster than one tile per workgroup.
+      if (t.id == LR_TILE_256x256 && streamed && s == 1 && tiles >= 2 * cus) us *= 0.985;
+      if (best_us == 0.0 || us < best_us) best_us = us, best = Plan{t.id, s};
+    }
   }
-  if (tile == LR_TILE_AUTO && pl.tile == LR_TILE_256x256 && pl.splits == 1 &&
-      (epilogue == LR_EPI_BF16 || epilogue == LR_EPI_GELU_TANH) && k % 128 == 0 && k >= 256 &&
-      ((m + 255) / 256) * ((n + 255) / 256) >= 2 * (int64_t)compute_units())
-    pl.tile = LR_TILE_256x256_PERSISTENT;
-  return pl;
+  return best;
 }
 
-int64_t split_workspace(int64_t m, int64_t n, int splits) { return splits > 1 ? splits * m * n * 4 : 0; }
+// The fast-path schedule. tile LR_TILE_AUTO: by the model above (K % 128 != 0: by
+// the rules of ragged_tile, unsplit), and where the model
+// takes 256x256 tiles over at least two waves of the chip and the epilogue is
+// bf16 or GELU, the persistent grid with streamed tiles, 1-2% faster than one
+// tile per workgroup (QKV 12288x15360x5120: 660 against 672 us, FFN-up 894
+// against 902-914 us, the Flash model's QKV and out-proj shapes at full M
+// likewise; same box). Its pass-staged gated epilogue is slower (out-proj 286
+// against 265 us), so the gated and raw epilogues keep one tile per workgroup.
+// workspace_bytes: what an automatic split may use.
+//
+// The search takes about 2 us, so each thread keeps its last results by shape
+// (a function of the arguments and the device's CU count alone).
+Plan plan(int64_t m, int64_t n, int64_t k, int tile, int splits, int64_t workspace_bytes, int epilogue) {
+  if (tile != LR_TILE_AUTO) return Plan{tile, splits > 0 ? splits : 1};
+  if (k % 128 != 0) return Plan{ragged_tile(m, n, k), splits > 0 ? splits : 1};
+  const bool streamed = (epilogue == LR_EPI_BF16 || epilogue == LR_EPI_GELU_TANH) && k >= 256;
+  struct Entry {
+    int64_t m, n, k, bytes;
+    int splits, cus;
+    bool streamed;
+    Plan plan;
+  };
+  constexpr int kEntries = 64;
+  static thread_local Entry cache[kEntries] = {};
+  const int64_t bytes = workspace_bytes < kAutoSliceBytes ? workspace_bytes : kAutoSliceBytes;
+  const int cus = compute_units();
+  const uint64_t h = (uint64_t)(m * 31 + n) * 0x9E3779B97F4A7C15ull ^ (uint64_t)(k * 8 + streamed * 4 + splits);
+  Entry& e = cache[(h ^ (h >> 29)) % kEntries];
+  if (e.m != m || e.n != n || e.k != k || e.bytes != bytes || e.splits != splits || e.cus != cus ||
+      e.streamed != streamed) {
+    e = Entry{m, n, k, bytes, splits, cus, streamed, search(m, n, k, splits, bytes, streamed)};
+    if (streamed && e.plan.tile == LR_TILE_256x256 && e.plan.splits == 1 &&
+        ((m + 255) / 256) * ((n + 255) / 256) >= 2 * (int64_t)cus)
+      e.plan.tile = LR_TILE_256x256_PERSISTENT;
+  }
+  return e.plan;
+}
 
 int gemm_impl(const int8_t* a, const int8_t* b, int64_t b_stride_k, int64_t b_stride_n, int64_t m,
               int64_t n, int64_t k, const float* row_scale, const float* col_scale, const void* bias,
@@ -1565,7 +1677,7 @@ int gemm_impl(const int8_t* a, const int8_t* b, int64_t b_stride_k, int64_t b_st
   LR_REQUIRE(m >= 0 && n >= 0 && k >= 0, "int8_gemm: negative shape");
   LR_REQUIRE(epilogue >= LR_EPI_BF16 && epilogue <= LR_EPI_RAW_INT32,
              "int8_gemm: unknown epilogue %d", epilogue);
-  LR_REQUIRE(tile >= LR_TILE_AUTO && tile <= LR_TILE_256x256_PERSISTENT, "int8_gemm: unknown tile %d",
+  LR_REQUIRE(tile >= LR_TILE_AUTO && tile <= LR_TILE_LAST, "int8_gemm: unknown tile %d",
              tile);
   LR_REQUIRE(splits >= 0 && splits <= 64, "int8_gemm: splits %d outside 0..64", splits);
   LR_REQUIRE(workspace_bytes >= 0 && (workspace != nullptr || workspace_bytes == 0),
@@ -1605,7 +1717,9 @@ int gemm_impl(const int8_t* a, const int8_t* b, int64_t b_stride_k, int64_t b_st
     LR_REQUIRE((m + 63) / 64 <= 65535, "int8_gemm: generic path supports M <= 4194240");
     LR_REQUIRE(splits <= 1, "int8_gemm: split-K needs the MFMA fast path");
   } else {
-    const Plan pl = plan(m, n, k, tile, splits, workspace != nullptr, epilogue);
+    // An automatic split uses what the workspace holds; a forced one needs its size.
+    const Plan pl = plan(m, n, k, tile, splits, workspace && aligned(workspace, 256) ? workspace_bytes : 0,
+                         epilogue);
     tile = pl.tile;
     const int64_t tiles = ((m + tile_rows(tile) - 1) / tile_rows(tile)) *
                           ((n + tile_cols(tile) - 1) / tile_cols(tile));
@@ -1727,6 +1841,9 @@ extern "C" int lr_int8_gemm_noalloc(const int8_t* a, const int8_t* b, int64_t b_
                                     int64_t sequence, int gate_slot, int splits, int tile,
                                     void* stream) {
   LR_REQUIRE(splits >= 0 && splits <= 64, "int8_gemm: splits %d outside 0..64", splits);
+  // Calls that overlap share the scratch and race, so an automatic split is
+  // taken only where it gains most (a few hundred rows at long K).
+  if (splits == 0 && !(m <= 256 && k >= 16384)) splits = 1;
   const int64_t need = m > 0 && n > 0 && k > 0 ? lr_int8_gemm_workspace_size(m, n, k, splits, tile) : 0;
   LR_REQUIRE(need <= kScratchBytes,
              "int8_gemm_noalloc: this split needs %lld bytes of scratch, above the %lld-byte maximum "
@@ -1744,7 +1861,7 @@ extern "C" int lr_int8_gemm_noalloc(const int8_t* a, const int8_t* b, int64_t b_
 
 extern "C" int64_t lr_int8_gemm_workspace_size(int64_t m, int64_t n, int64_t k, int splits, int tile) {
   if (m <= 0 || n <= 0 || k <= 0 || k % 128 != 0 || n % 4 != 0 || splits < 0 || splits > 64 ||
-      tile < LR_TILE_AUTO || tile > LR_TILE_256x256_PERSISTENT || tile == LR_TILE_GENERIC)
+      tile < LR_TILE_AUTO || tile > LR_TILE_LAST || tile == LR_TILE_GENERIC)
     return 0;
-  return split_workspace(m, n, plan(m, n, k, tile, splits, true, LR_EPI_RAW_INT32).splits);
+  return split_workspace(m, n, plan(m, n, k, tile, splits, kAutoSliceBytes, LR_EPI_RAW_INT32).splits);
 }

@@ -44,6 +44,11 @@ _TILES = {
     (64, 80): _lib.TILE_64x80,
     (128, 160): _lib.TILE_128x160,
     (192, 256): _lib.TILE_192x256,
+    (224, 256): _lib.TILE_224x256,
+    (160, 256): _lib.TILE_160x256,
+    (192, 128): _lib.TILE_192x128,
+    (128, 192): _lib.TILE_128x192,
+    (96, 128): _lib.TILE_96x128,
 }
 
 
@@ -110,7 +115,8 @@ def _launch(a, b, row_scale, column_scale, bias, out, epilogue, tile, residual=N
 # The candidates: every HIP tile, the library's own choice first, so that a
 # tie keeps it.
 _CANDIDATES = (None, (256, 256), "persistent", (192, 256), (256, 192), (256, 128), (128, 256),
-               (128, 128), (64, 128), (256, 80), (128, 160), (64, 80))
+               (128, 128), (64, 128), (256, 80), (128, 160), (64, 80), (224, 256), (160, 256),
+               (192, 128), (128, 192), (96, 128))
 _selected: dict[tuple, object] = {}
 _prefixes: dict[int, tuple] = {}
 

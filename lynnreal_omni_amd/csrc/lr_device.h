@@ -61,10 +61,17 @@ __device__ __forceinline__ uint4 buf_load16_reused(__amdgpu_buffer_rsrc_t r, uin
 // write-back lands in the GEMM that follows.
 constexpr int kStore16Policy = 0x11;  // sc0 | sc1
 constexpr int kStore8Policy = 0x2;    // nt
+// gfx950 reads the data registers of a store past 64 bits late, and the
+// compiler keeps the next instructions from overwriting them only where the
+// offset is not an SGPR. With one, a v_lshlrev right behind the store zeroed
+// the first word of a few lanes' data (bf16 norm rows wider than 5120, a few
+// hundred elements in 12605 rows of 5376). The wait below reads the data, so
+// whatever overwrites it comes two wait states after the store.
 __device__ __forceinline__ void buf_store16(__amdgpu_buffer_rsrc_t r, uint32_t voff,
                                             uint32_t soff, uint4 v) {
   const v4u w = {v.x, v.y, v.z, v.w};
   __builtin_amdgcn_raw_buffer_store_b128(w, r, voff, soff, kStore16Policy);
+  if (!(__builtin_constant_p(soff) && soff == 0)) asm volatile("s_nop 1" ::"v"(w));
 }
 __device__ __forceinline__ void buf_store8(__amdgpu_buffer_rsrc_t r, uint32_t voff,
                                            uint32_t soff, uint2 v) {

@@ -358,6 +358,7 @@ __device__ __forceinline__ void norm_row_f32(const NormArgs& p, int64_t row, con
   float ms = ss / (float)H;
   ms = ms + p.eps;
   const float rr = 1.0f / __builtin_sqrtf(ms);
+  const auto orow = row_rsrc(p.out + row * H, 2 * H);
   float amax = 0.0f;
 #pragma unroll
   for (int m = 0; m < CPL; ++m) {
@@ -373,6 +374,7 @@ __device__ __forceinline__ void norm_row_f32(const NormArgs& p, int64_t row, con
       f[m][e] = round_bf(t + sh[e]);
       amax = fmaxf(amax, __builtin_fabsf(f[m][e]));
     }
+    if (!QUANT) buf_store16(orow, 16u * lane, 1024u * m, pack8(f[m]));
     __builtin_amdgcn_sched_barrier(0);
   }
   if (QUANT) {
@@ -396,10 +398,6 @@ __device__ __forceinline__ void norm_row_f32(const NormArgs& p, int64_t row, con
       }
     }
     if (lane == 0) p.scales[row] = s;
-  } else {
-    const auto orow = row_rsrc(p.out + row * H, 2 * H);
-#pragma unroll
-    for (int m = 0; m < CPL; ++m) buf_store16(orow, 16u * lane, 1024u * m, pack8(f[m]));
   }
 }
 

@@ -3,8 +3,9 @@
 // Restates model/kernels.py:48-128 (_rms_adaln_kernel and
 // _rms_adaln_quant_int8_kernel, incl. its WITH_RESIDUAL branch :101-105).
 //
-// Main kernel: one wave per row (token), four rows per 256-thread block, no
-// block barriers. Lane l holds 16-byte chunks l, l+64, ... of the row in
+// Many rows: a persistent grid, one wave per row (rms_adaln_stream); few rows, or
+// rows with a residual: one row per 256-thread block (rms_adaln_row). Lane l
+// (thread t) holds 16-byte chunks l, l+64, ... (t, t+256, ...) of the row in
 // registers from the first read to the last write, so HBM sees each byte once:
 //   rms_adaln            2 B in + 2 B out per element
 //   rms_adaln_quant      2 B in + 1 B out per element (+4 B/row)
@@ -21,8 +22,8 @@
 // The reference's Triton kernel sums in its own tree order with an
 // approximate rsqrt; against it the bf16 outputs agree to a bf16 ulp.
 //
-// Rows wider than the wave kernel holds (hidden > 8192) or unaligned rows use
-// a one-row-per-block kernel with the same arithmetic.
+// Rows wider than 8192 or unaligned rows use a general one-row-per-block kernel
+// with the same arithmetic.
 #include "lr_device.h"
 #include "lr_runtime.h"
 
@@ -86,6 +87,15 @@ __device__ __forceinline__ void store8_i8(int8_t* row, int64_t c, int64_t n, con
       if (i < n) row[i] = (int8_t)quant_one(f[e], s, inv);
     }
   }
+}
+
+// A block barrier that leaves global loads in flight.
+__device__ __forceinline__ void lds_barrier() {
+  __builtin_amdgcn_sched_barrier(0);
+  __builtin_amdgcn_s_waitcnt(0xc07f);  // lgkmcnt(0): this wave's LDS accesses are done
+  __builtin_amdgcn_s_barrier();
+  asm volatile("" ::: "memory");
+  __builtin_amdgcn_sched_barrier(0);
 }
 
 template <int CPT, bool VEC, bool RESID, bool QUANT>
@@ -176,16 +186,19 @@ __global__ __launch_bounds__(kThreads) void rms_adaln_kernel(NormArgs p) {
 // global memory. Slices are ceil(rows / resident blocks) rows, so every CU
 // gets the same share whatever the frame length.
 // Waves per block: 16 (four per SIMD, one row per wave at a time) for rows up
-// to 5120 wide without a residual, else 8 (two rows per wave, the next one's
-// loads in flight). The LDS block is per block, so more waves per block share it.
+// to 5632 wide without a residual, 12 up to 6144, else 8 (two rows per wave, the
+// next one's loads in flight). The LDS block is per block, so more waves per block
+// share it.
 template <int CPL, bool RESID>
-constexpr int stream_waves() { return (RESID || CPL > 10) ? 8 : 16; }
+constexpr int stream_waves() { return RESID || CPL > 12 ? 8 : CPL > 11 ? 12 : 16; }
 
-// Rows up to 5120 wide without a residual: one row in registers per wave and
-// four waves per SIMD (108 VGPRs) hide the loads better than two rows per
-// wave at three waves per SIMD (measured 2% faster on the C2 shape).
+// Rows up to 6144 wide without a residual: one row in registers per wave and
+// four waves per SIMD (three past 5632; 108-142 VGPRs) hide the loads better than
+// two rows per wave at three waves per SIMD (5120 wide, 12288 rows: 2% faster).
+// Against the one-row-per-block kernel that the widths past 5120 ran before
+// (12605 x 5376, 6 table rows): 55.5 -> 47.3 us.
 template <int CPL, bool RESID>
-constexpr bool single_buffer() { return !RESID && CPL <= 10; }
+constexpr bool single_buffer() { return !RESID && CPL <= 12; }
 
 // LDS: parameter array a (0 gamma, 1 bf16(1 + scale), 2 shift, 3 gate),
 // chunk c, half h (elements 8c + 4h .. 8c + 4h + 3) at float4 (2a + h) * cap + c,
@@ -505,6 +518,133 @@ __global__ __launch_bounds__((64 * stream_waves<CPL, RESID>())) void rms_adaln_s
   }
 }
 
+// --------------------------------------------------- one row per block ----
+// Thread t holds chunks t, t + 256, ... (slot t of the sum of squares). Every load
+// of the row, the gate, gamma, scale and shift among them, is issued before
+// the first is used, through descriptors that end with the row, so a row waits
+// for memory once.
+template <int CPT, bool RESID, bool QUANT, bool NT>
+__global__ __launch_bounds__(kThreads) void rms_adaln_row(NormArgs p) {
+  __shared__ float slots[kThreads];
+  __shared__ float maxima[4];
+  const int64_t H = p.hidden;
+  const int64_t row = blockIdx.x;
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+  const uint32_t off = 16u * threadIdx.x;
+  auto load = [&](const uint16_t* src, uint4 (&v)[CPT]) {
+    const auto r = row_rsrc(src, 2 * H);
+#pragma unroll
+    for (int i = 0; i < CPT; ++i) v[i] = buf_load16_reused(r, off, 4096u * i);
+  };
+  uint4 xv[CPT], uv[RESID ? CPT : 1], wv[CPT], modv[CPT], shv[CPT], gv[RESID ? CPT : 1];
+  const auto rx = row_rsrc(p.x + row * H, 2 * H);
+#pragma unroll
+  for (int i = 0; i < CPT; ++i)
+    xv[i] = NT ? buf_load16(rx, off, 4096u * i) : buf_load16_reused(rx, off, 4096u * i);
+  if constexpr (RESID) {
+    const auto ru = row_rsrc(p.u + row * H, 2 * H);
+#pragma unroll
+    for (int i = 0; i < CPT; ++i)
+      uv[i] = NT ? buf_load16(ru, off, 4096u * i) : buf_load16_reused(ru, off, 4096u * i);
+  }
+  // One table row needs no index, and one sequence no division.
+  int64_t tr = 0;
+  if (p.table_rows > 1)
+    tr = clamp_index(p.indices[row < p.sequence ? row : row % p.sequence], p.table_rows);
+  const uint16_t* trow = p.table + tr * p.table_width;
+  if constexpr (RESID) load(trow + 2 * H, gv);
+  load(p.w, wv);
+  load(trow + (int64_t)p.scale_slot * H, modv);
+  load(trow + (int64_t)p.shift_slot * H, shv);
+  __builtin_amdgcn_sched_barrier(0);
+
+  float f[CPT][8];
+#pragma unroll
+  for (int i = 0; i < CPT; ++i) unpack8(xv[i], f[i]);
+  if constexpr (RESID) {
+    // x' = bf16(x + bf16(gate * u)), gate = table slot 2 (kernels.py:101-105)
+    const auto rr_ = row_rsrc(p.resid_out + row * H, 2 * H);
+#pragma unroll
+    for (int i = 0; i < CPT; ++i) {
+      float g[8], u[8];
+      unpack8(gv[i], g);
+      unpack8(uv[i], u);
+#pragma unroll
+      for (int e = 0; e < 8; ++e) f[i][e] = f[i][e] + round_bf(g[e] * u[e]);
+      const uint4 packed = pack8(f[i]);
+      unpack8(packed, f[i]);
+      buf_store16(rr_, off, 4096u * i, packed);
+    }
+  }
+  // A bf16 square is exact in fp32, so fma(x, x, s) is s + x*x rounded once.
+  float acc = 0.0f;
+#pragma unroll
+  for (int i = 0; i < CPT; ++i)
+#pragma unroll
+    for (int e = 0; e < 8; ++e) acc = __builtin_fmaf(f[i][e], f[i][e], acc);
+  slots[threadIdx.x] = acc;
+  lds_barrier();
+  const float ss = wave_tree_sum((slots[lane] + slots[lane + 128]) + (slots[lane + 64] + slots[lane + 192]));
+  float ms = ss / (float)H;
+  ms = ms + p.eps;
+  const float rr = 1.0f / __builtin_sqrtf(ms);
+  const auto orow = row_rsrc(p.out + row * H, 2 * H);
+  float amax = 0.0f;
+#pragma unroll
+  for (int i = 0; i < CPT; ++i) {
+    float w[8], sc[8], sh[8];
+    unpack8(wv[i], w);
+    unpack8(modv[i], sc);
+    unpack8(shv[i], sh);
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+      const float n = round_bf((f[i][e] * rr) * w[e]);
+      const float m = round_bf(n * round_bf(1.0f + sc[e]));
+      f[i][e] = round_bf(m + sh[e]);
+      amax = fmaxf(amax, __builtin_fabsf(f[i][e]));
+    }
+    if (!QUANT) buf_store16(orow, off, 4096u * i, pack8(f[i]));
+  }
+  if constexpr (QUANT) {
+    amax = wave_max(amax);
+    if (lane == 0) maxima[wave] = amax;
+    lds_barrier();
+    amax = fmaxf(fmaxf(maxima[0], maxima[1]), fmaxf(maxima[2], maxima[3]));
+    const float s = quant_scale(amax);
+    const float inv = 1.0f / s;
+    const auto qrow = row_rsrc(p.q + row * H, H);
+    if (__builtin_amdgcn_readfirstlane(amax < 0x1p80f ? 1 : 0)) {  // the three-operation quotient
+      const float lo = quant_lo(s, inv);
+#pragma unroll
+      for (int i = 0; i < CPT; ++i)
+        buf_store8(qrow, 8u * threadIdx.x, 2048u * i, quant8_split(f[i], inv, lo));
+    } else {
+#pragma unroll
+      for (int i = 0; i < CPT; ++i) buf_store8(qrow, 8u * threadIdx.x, 2048u * i, quant8(f[i], s, inv));
+    }
+    if (threadIdx.x == 0) p.scales[row] = s;
+  }
+}
+
+template <bool RESID, bool QUANT, bool NT>
+void launch_row(const NormArgs& p, int64_t rows, hipStream_t st) {
+  const dim3 grid((unsigned)rows), block(kThreads);
+  const int64_t chunks = p.hidden / 8;
+  if (chunks <= 256) hipLaunchKernelGGL((rms_adaln_row<1, RESID, QUANT, NT>), grid, block, 0, st, p);
+  else if (chunks <= 512) hipLaunchKernelGGL((rms_adaln_row<2, RESID, QUANT, NT>), grid, block, 0, st, p);
+  else if (chunks <= 768) hipLaunchKernelGGL((rms_adaln_row<3, RESID, QUANT, NT>), grid, block, 0, st, p);
+  else hipLaunchKernelGGL((rms_adaln_row<4, RESID, QUANT, NT>), grid, block, 0, st, p);
+}
+
+// Inputs of up to 24 MB are read through the caches, where the kernel that
+// produced them left them (residual norm of 878 x 5376 9.4 against 10.8 us
+// non-temporal); larger ones non-temporally (12605 rows 85.3 against 91.6 us).
+template <bool RESID, bool QUANT>
+void launch_norm_row(const NormArgs& p, int64_t rows, hipStream_t st) {
+  if (rows * p.hidden * 2 > 24LL << 20) launch_row<RESID, QUANT, true>(p, rows, st);
+  else launch_row<RESID, QUANT, false>(p, rows, st);
+}
+
 template <int CPL, bool RESID, bool QUANT>
 void launch_stream(const NormArgs& p, int64_t rows, hipStream_t st) {
   constexpr int kStreamWaves = stream_waves<CPL, RESID>();
@@ -527,8 +667,9 @@ void launch_stream(const NormArgs& p, int64_t rows, hipStream_t st) {
                      per_block);
 }
 
-// Rows up to 5120 wide (8192 without quantization) stay in registers without
-// spilling; wider rows take the one-row-per-block kernel.
+// False where the row's width has no streaming kernel that keeps it in
+// registers (quantizing rows wider than 6144, rows with a residual wider than
+// 3072, which the row kernel runs faster anyway).
 template <bool RESID, bool QUANT>
 bool launch_norm_stream(const NormArgs& p, int64_t rows, hipStream_t st) {
   const int64_t need = (p.hidden / 8 + 63) / 64;
@@ -536,38 +677,56 @@ bool launch_norm_stream(const NormArgs& p, int64_t rows, hipStream_t st) {
   else if (need <= 2) launch_stream<2, RESID, QUANT>(p, rows, st);
   else if (need <= 4) launch_stream<4, RESID, QUANT>(p, rows, st);
   else if (need <= 6) launch_stream<6, RESID, QUANT>(p, rows, st);
-  else if (need <= 8) launch_stream<8, RESID, QUANT>(p, rows, st);
-  else if (need <= 10) launch_stream<10, RESID, QUANT>(p, rows, st);
+  else if (RESID) return false;
+  else if (need <= 8) launch_stream<8, false, QUANT>(p, rows, st);
+  else if (need <= 10) launch_stream<10, false, QUANT>(p, rows, st);
+  else if (need <= 11) launch_stream<11, false, QUANT>(p, rows, st);
+  else if (need <= 12) launch_stream<12, false, QUANT>(p, rows, st);
   else if (QUANT) return false;
-  else if (need <= 12) launch_stream<12, false, false>(p, rows, st);
   else if (need <= 16) launch_stream<16, false, false>(p, rows, st);
   else return false;
   return true;
 }
 
+// One row per block, or a persistent grid that stages its parameters once: the
+// staging (and, with several table rows, the search for their boundaries) costs
+// 3-6 us, which many rows repay and few do not. us, graph-replayed, one row per
+// block / streamed: norm + quant of 878 x 5376, 6 table rows 7.3 / 11.7, 3683
+// rows 17.6 / 19.3, 6144 rows 26.7 / 24.3, 12605 rows 51.6 / 47.3; one table row
+// 878 rows 7.0 / 7.5, 2048 rows 11.4 / 10.2; narrow rows cross earlier (1024 wide,
+// 6 table rows: 4096 rows 9.6 / 9.6). With a residual the row kernel has 5 blocks
+// per CU in flight where the streamed one has 8 waves of two rows each, and is
+// ahead at every count from 3072 columns on (12605 x 5120 82.5 / 87.4, 512 x 5120
+// 6.8 / 14.8); below, up to the counts here (2048 wide: 6144 rows 19.8 / 21.5).
+bool prefer_row_kernel(bool resid, int64_t rows, int64_t hidden, int64_t table_rows) {
+  if (resid) return hidden > 3072 || rows < (hidden >= 2048 ? 8192 : 3072);
+  if (table_rows == 1) return rows < (hidden > 3072 ? 1536 : 1024);
+  return rows < (hidden > 1024 ? 4096 : 2560);
+}
+
 template <bool RESID, bool QUANT>
 int launch_norm(const NormArgs& p, int64_t rows, bool vec, hipStream_t st) {
-  if (vec && launch_norm_stream<RESID, QUANT>(p, rows, st)) return check_launch("rms_adaln");
   const int64_t chunks = (p.hidden + 7) / 8;
+  if (vec && chunks <= 1024) {
+    if (prefer_row_kernel(RESID, rows, p.hidden, p.table_rows) || !launch_norm_stream<RESID, QUANT>(p, rows, st))
+      launch_norm_row<RESID, QUANT>(p, rows, st);
+    return check_launch("rms_adaln");
+  }
   const int64_t need = (chunks + kThreads - 1) / kThreads;
   if (need > 16)
     return fail(LR_EUNSUPPORTED, "rms_adaln: hidden=%lld not supported (max %d)",
                 (long long)p.hidden, 16 * 8 * kThreads);
-#define LR_NORM_LAUNCH(C)                                                                   \
-  do {                                                                                      \
-    if (vec)                                                                                \
-      hipLaunchKernelGGL((rms_adaln_kernel<C, true, RESID, QUANT>), dim3((unsigned)rows),   \
-                         dim3(kThreads), 0, st, p);                                         \
-    else                                                                                    \
-      hipLaunchKernelGGL((rms_adaln_kernel<C, false, RESID, QUANT>), dim3((unsigned)rows),  \
-                         dim3(kThreads), 0, st, p);                                         \
-  } while (0)
-  if (need <= 1) LR_NORM_LAUNCH(1);
-  else if (need <= 2) LR_NORM_LAUNCH(2);
-  else if (need <= 3) LR_NORM_LAUNCH(3);
-  else if (need <= 4) LR_NORM_LAUNCH(4);
-  else if (need <= 8) LR_NORM_LAUNCH(8);
-  else LR_NORM_LAUNCH(16);
+#define LR_NORM_LAUNCH(C, V)                                                                  \
+  hipLaunchKernelGGL((rms_adaln_kernel<C, V, RESID, QUANT>), dim3((unsigned)rows), dim3(kThreads), \
+                     0, st, p)
+  if (vec && need <= 8) LR_NORM_LAUNCH(8, true);
+  else if (vec) LR_NORM_LAUNCH(16, true);
+  else if (need <= 1) LR_NORM_LAUNCH(1, false);
+  else if (need <= 2) LR_NORM_LAUNCH(2, false);
+  else if (need <= 3) LR_NORM_LAUNCH(3, false);
+  else if (need <= 4) LR_NORM_LAUNCH(4, false);
+  else if (need <= 8) LR_NORM_LAUNCH(8, false);
+  else LR_NORM_LAUNCH(16, false);
 #undef LR_NORM_LAUNCH
   return check_launch("rms_adaln");
 }

@@ -53,3 +53,25 @@ def test_quantizing_norms_equal_their_two_steps(rows, hidden):
         r0 = k._gated_residual(x, u, table, indices, 2)
         q0, s0 = k._rms_adaln_quant_int8(r0, norm, table, indices, 3, 4)
         assert torch.equal(r, r0) and torch.equal(q, q0) and torch.equal(s, s0)
+
+
+@pytest.mark.parametrize("table_rows", [1, 3])
+@pytest.mark.parametrize("hidden", [8, 2040, 2048, 2056, 4096, 4104, 6144, 6152, 8184, 8192])
+def test_row_kernel_edges(hidden, table_rows):
+    """One row per block at the edges of its chunk counts, two sequences (rows
+    past the first index by row modulo the sequence), against the oracle."""
+    import gpu_adapter as gpu
+    from helpers import bf16_randn, to_np
+    from oracle import reference as ref
+
+    g = torch.Generator().manual_seed(hidden + table_rows)
+    x, u = (to_np(bf16_randn((2, 3, hidden), g, outliers=0.01)) for _ in range(2))
+    w = to_np((1 + 0.05 * torch.randn(hidden, generator=g)).bfloat16())
+    table = to_np(bf16_randn((table_rows, 6 * hidden), g, scale=0.1))
+    idx = torch.randint(0, table_rows, (3,), generator=g).numpy()
+    args = (x, w, table, idx)
+    assert (gpu.rms_adaln(*args, 0, 1, 1e-6) == ref.rms_adaln(*args, 0, 1, 1e-6)).all()
+    for got, want in ((gpu.rms_adaln_quant(*args, 3, 4, 1e-6), ref.rms_adaln_quant(*args, 3, 4, 1e-6)),
+                      (gpu.residual_rms_quant(x, u, w, table, idx, 1e-6),
+                       ref.residual_rms_quant(x, u, w, table, idx, 1e-6))):
+        assert all((a == b).all() for a, b in zip(got, want))

@@ -79,6 +79,12 @@ __device__ __forceinline__ void buf_store8(__amdgpu_buffer_rsrc_t r, uint32_t vo
   __builtin_amdgcn_raw_buffer_store_b64(w, r, voff, soff, kStore8Policy);
 }
 
+__device__ __forceinline__ void buf_store8_cached(__amdgpu_buffer_rsrc_t r, uint32_t voff,
+                                                  uint32_t soff, uint2 v) {
+  const v2u w = {v.x, v.y};
+  __builtin_amdgcn_raw_buffer_store_b64(w, r, voff, soff, 0);
+}
+
 // ---------------------------------------------------------------- bf16 ----
 __device__ __forceinline__ float bf_lo(uint32_t w) { return __uint_as_float(w << 16); }
 __device__ __forceinline__ float bf_hi(uint32_t w) { return __uint_as_float(w & 0xffff0000u); }

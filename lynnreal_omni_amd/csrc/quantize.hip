@@ -2,11 +2,11 @@
 // INT32 -> bf16 dequant epilogue.
 //
 // quantize_rows restates model/int8.py:66-67 (the torch path; the Triton
-// kernel model/kernels.py:8-16 computes the same values). Rows up to 8192
-// wide: one wave per row, four rows per 256-thread block; lane l holds 16-byte
+// kernel model/kernels.py:8-16 computes the same values). Narrow rows (under
+// 4096): one wave per row, four rows per 256-thread block; lane l holds 16-byte
 // chunks l, l+64, ... in registers, the absmax is a wave butterfly, and the
-// row is quantized from registers and written with 8-byte stores. Wider rows:
-// one 256-thread block per row, same scheme with a block reduction. HBM
+// row is quantized from registers and written with 8-byte stores. Wider or few
+// rows: one 256-thread block per row, same scheme with a block reduction. HBM
 // traffic is the algorithmic 3 bytes/element plus 4 bytes/row.
 #include "lr_device.h"
 #include "lr_runtime.h"
@@ -43,22 +43,26 @@ __global__ __launch_bounds__(kThreads) void quantize_rows_wave(const uint4* __re
   if (lane == 0) scales[row] = s;
 }
 
-template <int CPT>
-__global__ __launch_bounds__(kThreads) void quantize_rows_vec(const uint4* __restrict__ x,
-                                                              uint2* __restrict__ q,
-                                                              float* __restrict__ scales,
-                                                              int chunks) {
+// One block per row, for rows of 4096 and more and for few rows of any width,
+// where a wave per row has more serial work than it hides. Loads and stores go
+// through descriptors that end with the row. NT: non-temporal loads, for inputs
+// past 32 MB; smaller ones are still in the caches from the kernel that wrote
+// them. Rows past 8192 are stored write-back (20480 wide, 12605 rows 116.7
+// against 123.9 us non-temporal), narrower ones non-temporally.
+template <int CPT, bool NT>
+__global__ __launch_bounds__(kThreads) void quantize_rows_block(const uint4* __restrict__ x,
+                                                                uint2* __restrict__ q,
+                                                                float* __restrict__ scales,
+                                                                int64_t chunks) {
   __shared__ float red[4];
   const int64_t row = blockIdx.x;
-  const uint4* src = x + row * chunks;
-  uint2* dst = q + row * chunks;
+  const auto src = row_rsrc(x + row * chunks, 16 * chunks);
+  const auto dst = row_rsrc(q + row * chunks, 8 * chunks);
   uint4 v[CPT];
   float m = 0.0f;
 #pragma unroll
-  for (int i = 0; i < CPT; ++i) {
-    const int c = threadIdx.x + i * kThreads;
-    v[i] = c < chunks ? load_nt(src + c) : make_uint4(0, 0, 0, 0);
-  }
+  for (int i = 0; i < CPT; ++i)
+    v[i] = NT ? buf_load16(src, 16u * threadIdx.x, 4096u * i) : buf_load16_reused(src, 16u * threadIdx.x, 4096u * i);
 #pragma unroll
   for (int i = 0; i < CPT; ++i) m = absmax8(v[i], m);
   m = block256_max(m, red);
@@ -66,8 +70,10 @@ __global__ __launch_bounds__(kThreads) void quantize_rows_vec(const uint4* __res
   const float inv = 1.0f / s;
 #pragma unroll
   for (int i = 0; i < CPT; ++i) {
-    const int c = threadIdx.x + i * kThreads;
-    if (c < chunks) dst[c] = quant8_bf(v[i], s, inv);
+    const uint2 b = quant8_bf(v[i], s, inv);
+    if (CPT > 4) buf_store8_cached(dst, 8u * threadIdx.x, 2048u * i, b);
+    else buf_store8(dst, 8u * threadIdx.x, 2048u * i, b);
+    __builtin_amdgcn_sched_barrier(0);
   }
   if (threadIdx.x == 0) scales[row] = s;
 }
@@ -116,11 +122,32 @@ __global__ __launch_bounds__(kThreads) void quantize_rows_typed(const T* __restr
   if (threadIdx.x == 0) scales[row] = s;
 }
 
-template <int CPT>
-void launch_quant_vec(const void* x, int8_t* q, float* s, int64_t rows, int chunks,
-                      hipStream_t st) {
-  hipLaunchKernelGGL(quantize_rows_vec<CPT>, dim3((unsigned)rows), dim3(kThreads), 0, st,
+template <int CPT, bool NT>
+void launch_quant_block(const void* x, int8_t* q, float* s, int64_t rows, int64_t chunks,
+                        hipStream_t st) {
+  hipLaunchKernelGGL((quantize_rows_block<CPT, NT>), dim3((unsigned)rows), dim3(kThreads), 0, st,
                      (const uint4*)x, (uint2*)q, s, chunks);
+}
+
+// us, wave per row / block per row (graph-replayed, rotating inputs): 7168 wide,
+// 16 rows 4.1 / 2.5, 512 rows 4.8 / 3.8, 3683 rows 16.5 / 14.7, 12605 rows 45.5 /
+// 43.3; 5120 wide 256 rows 3.8 / 2.7, 12605 rows 32.5 / 31.6; 3072 wide 512 rows
+// 3.3 / 2.9, 12605 rows 20.1 / 21.8; 1024 wide slower at every count.
+void launch_quant_rows(const void* x, int8_t* q, float* s, int64_t rows, int64_t chunks,
+                       hipStream_t st) {
+  const int need = (int)((chunks + kThreads - 1) / kThreads);
+  if (rows * chunks * 16 <= 32LL << 20 && need <= 4) {
+    if (need <= 2) launch_quant_block<2, false>(x, q, s, rows, chunks, st);
+    else if (need <= 3) launch_quant_block<3, false>(x, q, s, rows, chunks, st);
+    else launch_quant_block<4, false>(x, q, s, rows, chunks, st);
+  } else if (need <= 2) launch_quant_block<2, true>(x, q, s, rows, chunks, st);
+  else if (need <= 3) launch_quant_block<3, true>(x, q, s, rows, chunks, st);
+  else if (need <= 4) launch_quant_block<4, true>(x, q, s, rows, chunks, st);
+  else if (need <= 6) launch_quant_block<6, true>(x, q, s, rows, chunks, st);
+  else if (need <= 8) launch_quant_block<8, true>(x, q, s, rows, chunks, st);
+  else if (need <= 10) launch_quant_block<10, true>(x, q, s, rows, chunks, st);
+  else if (need <= 12) launch_quant_block<12, true>(x, q, s, rows, chunks, st);
+  else launch_quant_block<16, true>(x, q, s, rows, chunks, st);
 }
 
 template <int CPL>
@@ -186,7 +213,9 @@ extern "C" int lr_quantize_rows(const void* x, int64_t rows, int64_t width, int8
   const int64_t chunks = width / 8;
   const bool vec = width % 8 == 0 && aligned(x, 16) && aligned(q, 8) && chunks <= 16 * kThreads &&
                    width > 0;
-  if (vec && chunks <= 16 * 64) {
+  if (vec && (chunks >= 512 || (chunks > 256 && rows <= 512))) {
+    launch_quant_rows(x, q, scales, rows, chunks, st);
+  } else if (vec) {
     const int need = (int)((chunks + 63) / 64);
     const int c = (int)chunks;
     if (need <= 1) launch_quant_wave<1>(x, q, scales, rows, c, st);
@@ -194,22 +223,7 @@ extern "C" int lr_quantize_rows(const void* x, int64_t rows, int64_t width, int8
     else if (need <= 3) launch_quant_wave<3>(x, q, scales, rows, c, st);
     else if (need <= 4) launch_quant_wave<4>(x, q, scales, rows, c, st);
     else if (need <= 6) launch_quant_wave<6>(x, q, scales, rows, c, st);
-    else if (need <= 8) launch_quant_wave<8>(x, q, scales, rows, c, st);
-    else if (need <= 10) launch_quant_wave<10>(x, q, scales, rows, c, st);
-    else if (need <= 12) launch_quant_wave<12>(x, q, scales, rows, c, st);
-    else launch_quant_wave<16>(x, q, scales, rows, c, st);
-  } else if (vec) {
-    const int need = (int)((chunks + kThreads - 1) / kThreads);
-    const int c = (int)chunks;
-    if (need <= 1) launch_quant_vec<1>(x, q, scales, rows, c, st);
-    else if (need <= 2) launch_quant_vec<2>(x, q, scales, rows, c, st);
-    else if (need <= 3) launch_quant_vec<3>(x, q, scales, rows, c, st);
-    else if (need <= 4) launch_quant_vec<4>(x, q, scales, rows, c, st);
-    else if (need <= 6) launch_quant_vec<6>(x, q, scales, rows, c, st);
-    else if (need <= 8) launch_quant_vec<8>(x, q, scales, rows, c, st);
-    else if (need <= 10) launch_quant_vec<10>(x, q, scales, rows, c, st);
-    else if (need <= 12) launch_quant_vec<12>(x, q, scales, rows, c, st);
-    else launch_quant_vec<16>(x, q, scales, rows, c, st);
+    else launch_quant_wave<8>(x, q, scales, rows, c, st);
   } else {
     hipLaunchKernelGGL(quantize_rows_any, dim3((unsigned)rows), dim3(kThreads), 0, st,
                        (const uint16_t*)x, q, scales, width);

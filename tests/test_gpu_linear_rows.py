@@ -44,3 +44,17 @@ def test_layer_and_its_errors():
         layer(x.cpu())
     with pytest.raises(ValueError, match="is on cpu"):
         int8_gemm.linear_rows(x[0], w.t(), layer.weight_scale, None)
+
+
+@pytest.mark.parametrize("rows", [1, 512, 513])
+@pytest.mark.parametrize("width", [2048, 2056, 4088, 4096, 4104, 6144, 6152, 8192, 8200, 12296])
+def test_quantizer_at_the_edges_of_its_kernels(rows, width):
+    """A wave and a block per row, at the widths and counts where one takes over
+    from the other and at their chunk counts, against the torch restatement."""
+    from oracle import torch_path as tp
+    g = torch.Generator().manual_seed(rows + width)
+    x = (torch.randn(rows, width, generator=g) * 5).bfloat16()
+    x[0] = 0
+    q, s = kernels.quantize_rows(x.cuda())
+    want_q, want_s = tp.quantize(x)
+    assert torch.equal(q.cpu(), want_q) and torch.equal(s.cpu().reshape(-1), want_s.reshape(-1))

@@ -1499,7 +1499,7 @@ struct AutoTile {
 };
 constexpr AutoTile kAutoTiles[] = {
     {LR_TILE_256x256, 256, 256, 1.0},    {LR_TILE_224x256, 224, 256, 1.0},
-    {LR_TILE_192x256, 192, 256, 0.96},   {LR_TILE_160x256, 160, 256, 1.0},
+    {LR_TILE_192x256, 192, 256, 1.0},   {LR_TILE_160x256, 160, 256, 1.0},
     {LR_TILE_256x128, 256, 128, 1.0},   {LR_TILE_128x256, 128, 256, 1.0},
     {LR_TILE_192x128, 192, 128, 0.97},  {LR_TILE_128x192, 128, 192, 1.0},
     {LR_TILE_128x160, 128, 160, 1.03},   {LR_TILE_96x128, 96, 128, 1.0},

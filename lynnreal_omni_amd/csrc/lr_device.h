@@ -73,6 +73,11 @@ __device__ __forceinline__ void buf_store16(__amdgpu_buffer_rsrc_t r, uint32_t v
   __builtin_amdgcn_raw_buffer_store_b128(w, r, voff, soff, kStore16Policy);
   if (!(__builtin_constant_p(soff) && soff == 0)) asm volatile("s_nop 1" ::"v"(w));
 }
+// Non-temporal, with the whole offset in `voff` (no SGPR offset, see above).
+__device__ __forceinline__ void buf_store16_nt(__amdgpu_buffer_rsrc_t r, uint32_t voff, uint4 v) {
+  const v4u w = {v.x, v.y, v.z, v.w};
+  __builtin_amdgcn_raw_buffer_store_b128(w, r, voff, 0, 2 /* nt */);
+}
 __device__ __forceinline__ void buf_store8(__amdgpu_buffer_rsrc_t r, uint32_t voff,
                                            uint32_t soff, uint2 v) {
   const v2u w = {v.x, v.y};

@@ -136,7 +136,9 @@ int lr_int8_gemm(const int8_t* a, const int8_t* b, int64_t b_stride_k, int64_t b
  * splits <= K / 128, N % 4 == 0). The library never allocates: workspace is
  * device memory of workspace_bytes >= lr_int8_gemm_workspace_size (256-byte
  * aligned), used only by the call's kernels on `stream`, so calls that share
- * one workspace must be ordered on one stream. With workspace NULL no split
+ * one workspace must be ordered on one stream. An automatic split takes what a
+ * smaller workspace holds, except for M <= 256 at K >= 16384, where one below
+ * the slices of a single wave of tiles is LR_EINVAL. With workspace NULL no split
  * is taken unless forced (then LR_EINVAL). Replaces the same reference
  * functions as lr_int8_gemm (model/int8_gemm.py:96-163, :13-46), whose Triton
  * autotuner covers small M with small tiles (model/int8_gemm.py:49-52). */
@@ -158,7 +160,7 @@ int64_t lr_int8_gemm_workspace_size(int64_t m, int64_t n, int64_t k, int splits,
  * No counterpart in the reference: it is for callers that cannot allocate
  * (code under HIP graph capture, tight serving loops, harnesses that forbid
  * hipMalloc). A split whose slices need more than 32 MiB is refused with
- * LR_EINVAL (the automatic choice needs at most about 21 MiB); calls that
+ * LR_EINVAL (the automatic choice needs at most 22 MiB); calls that
  * overlap on one GPU share the array and race. Same arguments, arithmetic
  * and outputs as lr_int8_gemm_ws. */
 int lr_int8_gemm_noalloc(const int8_t* a, const int8_t* b, int64_t b_stride_k, int64_t b_stride_n,

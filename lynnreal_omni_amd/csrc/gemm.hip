@@ -1603,6 +1603,16 @@ struct Plan {
 
 int64_t split_workspace(int64_t m, int64_t n, int splits) { return splits > 1 ? splits * m * n * 4 : 0; }
 
+// Slices that fill one wave of the CUs with 128x160 tiles, at most 4, for a few
+// hundred rows at long K, where a split gains most (256 x 5120 x 20480: 36 us,
+// 42 unsplit); 1 elsewhere. Bounds what an automatic split may take for granted,
+// not its choice.
+int long_k_slices(int64_t m, int64_t n, int64_t k) {
+  if (m <= 0 || n <= 0 || m > 256 || k < 16384 || k % 128 != 0 || n % 4 != 0) return 1;
+  const int64_t s = compute_units() / (((m + 127) / 128) * ((n + 159) / 160));
+  return s > 4 ? 4 : s > 1 ? (int)s : 1;
+}
+
 // The fastest (tile, splits) by the model, K % 128 == 0. splits 0: up to the workspace's
 // bytes; else that many. `streamed`: the epilogue can take the persistent grid
 // where 256x256 tiles make two waves of the chip or more.
@@ -1657,7 +1667,7 @@ Plan plan(int64_t m, int64_t n, int64_t k, int tile, int splits, int64_t workspa
   static thread_local Entry cache[kEntries] = {};
   const int64_t bytes = workspace_bytes < kAutoSliceBytes ? workspace_bytes : kAutoSliceBytes;
   const int cus = compute_units();
-  const uint64_t h = (uint64_t)(m * 31 + n) * 0x9E3779B97F4A7C15ull ^ (uint64_t)(k * 8 + streamed * 4 + splits);
+  const uint64_t h = (uint64_t)(m * 31 + n + bytes * 7) * 0x9E3779B97F4A7C15ull ^ (uint64_t)(k * 8 + streamed * 4 + splits);
   Entry& e = cache[(h ^ (h >> 29)) % kEntries];
   if (e.m != m || e.n != n || e.k != k || e.bytes != bytes || e.splits != splits || e.cus != cus ||
       e.streamed != streamed) {
@@ -1717,7 +1727,18 @@ int gemm_impl(const int8_t* a, const int8_t* b, int64_t b_stride_k, int64_t b_st
     LR_REQUIRE((m + 63) / 64 <= 65535, "int8_gemm: generic path supports M <= 4194240");
     LR_REQUIRE(splits <= 1, "int8_gemm: split-K needs the MFMA fast path");
   } else {
-    // An automatic split uses what the workspace holds; a forced one needs its size.
+    // An automatic split uses what the workspace holds; a forced one needs its
+    // size, and a few hundred rows at long K at least the smaller of one wave's
+    // slices and the choice's own.
+    if (splits == 0 && tile == LR_TILE_AUTO && workspace != nullptr) {
+      const int s = long_k_slices(m, n, k);
+      const int64_t wave = split_workspace(m, n, s);
+      const int64_t own = s == 1 ? 0 : lr_int8_gemm_workspace_size(m, n, k, 0, LR_TILE_AUTO);
+      const int64_t need = wave < own ? wave : own;
+      LR_REQUIRE(workspace_bytes >= need, "int8_gemm: %d-way split-K needs a %lld-byte workspace, got %lld", s,
+                 (long long)need, (long long)workspace_bytes);
+      LR_REQUIRE(s == 1 || aligned(workspace, 256), "int8_gemm: workspace must be 256-byte aligned");
+    }
     const Plan pl = plan(m, n, k, tile, splits, workspace && aligned(workspace, 256) ? workspace_bytes : 0,
                          epilogue);
     tile = pl.tile;
@@ -1842,8 +1863,8 @@ extern "C" int lr_int8_gemm_noalloc(const int8_t* a, const int8_t* b, int64_t b_
                                     void* stream) {
   LR_REQUIRE(splits >= 0 && splits <= 64, "int8_gemm: splits %d outside 0..64", splits);
   // Calls that overlap share the scratch and race, so an automatic split is
-  // taken only where it gains most (a few hundred rows at long K).
-  if (splits == 0 && !(m <= 256 && k >= 16384)) splits = 1;
+  // taken only where it gains most.
+  if (splits == 0 && long_k_slices(m, n, k) == 1) splits = 1;
   const int64_t need = m > 0 && n > 0 && k > 0 ? lr_int8_gemm_workspace_size(m, n, k, splits, tile) : 0;
   LR_REQUIRE(need <= kScratchBytes,
              "int8_gemm_noalloc: this split needs %lld bytes of scratch, above the %lld-byte maximum "

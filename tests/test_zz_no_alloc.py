@@ -82,3 +82,42 @@ def test_noalloc_forced_split_and_limit():
     assert rc == _lib.LR_EINVAL and b"maximum" in lib.lr_last_error()
     torch.cuda.synchronize()
     assert not out.any()
+
+
+def test_automatic_choice_takes_the_scratch_only_at_long_k():
+    """Calls whose automatic split is new with the workspace entry point (few
+    rows at short K, wide N at long K) leave the shared array alone: overlapping
+    noalloc calls stay independent there. The outputs are the same."""
+    lib = _lib.load()
+    streams = [torch.cuda.Stream() for _ in range(2)]
+    for m, n, k in ((32, 5376, 7168), (200, 20480, 16384)):
+        sets = [_inputs(m, n, k, seed) for seed in (5, 6)]
+        want = []
+        for a, w, rs, cs, bias in sets:
+            out = torch.empty(m, n, dtype=torch.bfloat16, device="cuda")
+            assert lib.lr_int8_gemm(*_args(a, w, rs, cs, bias, out, _lib.EPI_BF16), _lib.TILE_AUTO,
+                                    torch.cuda.current_stream().cuda_stream) == _lib.LR_OK
+            want.append(out)
+        got = [torch.empty_like(o) for o in want]
+        torch.cuda.synchronize()
+        for _ in range(8):
+            for (a, w, rs, cs, bias), out, st in zip(sets, got, streams):
+                assert lib.lr_int8_gemm_noalloc(*_args(a, w, rs, cs, bias, out, _lib.EPI_BF16), 0,
+                                                _lib.TILE_AUTO, st.cuda_stream) == _lib.LR_OK
+        torch.cuda.synchronize()
+        assert all(torch.equal(g, o) for g, o in zip(got, want)), (m, n, k)
+
+
+def test_long_k_workspace_below_its_slices_is_refused():
+    lib = _lib.load()
+    stream = torch.cuda.current_stream().cuda_stream
+    m, n, k = 256, 5120, 20480
+    a, w, rs, cs, bias = _inputs(m, n, k, 7)
+    out = torch.zeros(m, n, dtype=torch.bfloat16, device="cuda")
+    need = lib.lr_int8_gemm_workspace_size(m, n, k, 0, _lib.TILE_AUTO)
+    ws = torch.empty(need, dtype=torch.uint8, device="cuda")
+    rc = lib.lr_int8_gemm_ws(*_args(a, w, rs, cs, bias, out, _lib.EPI_BF16), ws.data_ptr(), 4096, 0,
+                             _lib.TILE_AUTO, stream)
+    assert rc == _lib.LR_EINVAL
+    torch.cuda.synchronize()
+    assert not out.any()

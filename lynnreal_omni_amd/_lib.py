@@ -191,9 +191,11 @@ _workspaces: dict[tuple[int, int], torch.Tensor] = {}
 _MAX_WORKSPACES = 16
 
 
-def workspace(t: torch.Tensor, nbytes: int) -> tuple[int | None, int]:
-    """(pointer, bytes) of a device workspace of at least `nbytes` for the
-    caller's current stream on t's device, or (None, 0) when none is needed.
+def workspace(t: torch.Tensor, nbytes: int) -> torch.Tensor | None:
+    """A device workspace of at least `nbytes` for the caller's current stream
+    on t's device, or None when none is needed. The caller holds it until its
+    kernels are launched: before that nothing orders them with a later use of
+    the memory.
 
     One buffer is kept per (device, stream), grown on demand, for the 16
     most recently used (device, stream) pairs: kernels that share a buffer
@@ -201,12 +203,11 @@ def workspace(t: torch.Tensor, nbytes: int) -> tuple[int | None, int]:
     buffer's memory to a later allocation on the same stream only, behind
     the work already queued there."""
     if nbytes <= 0:
-        return None, 0
+        return None
     if torch.cuda.is_current_stream_capturing():
         # Memory of the graph being captured: a kept buffer could be outgrown
         # and freed under the graph, or shared with another graph's replay.
-        buf = torch.empty(nbytes, dtype=torch.uint8, device=t.device)
-        return buf.data_ptr(), nbytes
+        return torch.empty(nbytes, dtype=torch.uint8, device=t.device)
     key = (t.get_device(), stream(t))
     buf = _workspaces.pop(key, None)
     if buf is None or buf.numel() < nbytes:
@@ -214,4 +215,4 @@ def workspace(t: torch.Tensor, nbytes: int) -> tuple[int | None, int]:
     _workspaces[key] = buf  # most recent last
     while len(_workspaces) > _MAX_WORKSPACES:
         _workspaces.pop(next(iter(_workspaces)))
-    return buf.data_ptr(), buf.numel()
+    return buf

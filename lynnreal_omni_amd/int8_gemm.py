@@ -98,7 +98,7 @@ def _launch(a, b, row_scale, column_scale, bias, out, epilogue, tile, residual=N
     tile_id = _lib.TILE_AUTO if tile is None else _tile_id(tile)
     splits = 0 if splits is None else int(splits)
     nbytes = _workspace_bytes(m, n, k, splits, tile_id)
-    ws, ws_bytes = _lib.workspace(a, nbytes) if nbytes else (None, 0)
+    ws = _lib.workspace(a, nbytes) if nbytes else None  # held until the launch
     sb0, sb1 = b.stride()
     _lib.call("lr_int8_gemm_ws", a.data_ptr(), b.data_ptr(), sb0, sb1, m, n, k,
               None if row_scale is None else row_scale.data_ptr(),
@@ -106,8 +106,9 @@ def _launch(a, b, row_scale, column_scale, bias, out, epilogue, tile, residual=N
               None if bias is None else bias.data_ptr(), out.data_ptr(), epilogue,
               None if residual is None else residual.data_ptr(),
               None if table is None else table.data_ptr(), table_rows, table_width,
-              None if indices is None else indices.data_ptr(), sequence, gate_slot, ws, ws_bytes,
-              splits, tile_id, _lib.stream(a))
+              None if indices is None else indices.data_ptr(), sequence, gate_slot,
+              None if ws is None else ws.data_ptr(), 0 if ws is None else ws.numel(), splits, tile_id,
+              _lib.stream(a))
     return out
 
 

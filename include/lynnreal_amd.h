@@ -67,7 +67,8 @@ extern "C" {
 #define LR_TILE_256x256_PERSISTENT 13 /* 256x256 on a persistent grid (one workgroup per CU looping
                                         over the tiles, each tile's last k-steps loading the next
                                         tile's first ones); replaces model/int8_tma.py:12-41 */
-/* Tiles between the large and the small-M ones: 8 waves on a 2x4 grid. */
+/* Tiles between the large and the small-M ones: 8 waves on a 2x4 grid, for
+ * K % 128 == 0. With another K they run LR_TILE_128x128 (the same outputs). */
 #define LR_TILE_224x256 14
 #define LR_TILE_160x256 15
 #define LR_TILE_192x128 16

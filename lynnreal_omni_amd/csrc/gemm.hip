@@ -1308,24 +1308,34 @@ struct FastCfg {
   int bm, bn;
 };
 
-// RAGGED = false: the tile has no kernel for K % 128 != 0; such calls run the
-// 128x128 tile (the same outputs), which the automatic choice never needs.
-template <int BM, int BN, int WAVES_M, int WAVES_N, int EPI, bool BIAS, int NA = GEMM_RING_A,
-          int NB = GEMM_RING_B, bool RAGGED = true>
-void launch_fast_cfg(GemmArgs& p, hipStream_t st) {
+// One tile per workgroup, for K % 128 == 0 (KALIGNED) or any K % 16 == 0.
+template <int BM, int BN, int WAVES_M, int WAVES_N, int EPI, bool BIAS, int NA, int NB, bool KALIGNED>
+void launch_tile(GemmArgs& p, hipStream_t st) {
   p.tiles_m = (int)((p.m + BM - 1) / BM);
   p.tiles_n = (int)((p.n + BN - 1) / BN);
   const unsigned grid = (unsigned)(p.tiles_m * p.tiles_n * p.splits);
-  constexpr bool kPingPong = GEMM_PINGPONG && WAVES_M * WAVES_N == 8;
-  if (p.k % 128 == 0) {
-    hipLaunchKernelGGL((gemm_fast<BM, BN, WAVES_M, WAVES_N, EPI, BIAS, NA, NB, true, kPingPong>),
-                       dim3(grid), dim3(64 * WAVES_M * WAVES_N), 0, st, p);
-  } else if constexpr (RAGGED) {
-    hipLaunchKernelGGL((gemm_fast<BM, BN, WAVES_M, WAVES_N, EPI, BIAS, NA, NB, false, false>),
-                       dim3(grid), dim3(64 * WAVES_M * WAVES_N), 0, st, p);
-  } else {
-    launch_fast_cfg<128, 128, 2, 2, EPI, BIAS>(p, st);
-  }
+  constexpr bool kPingPong = KALIGNED && GEMM_PINGPONG && WAVES_M * WAVES_N == 8;
+  hipLaunchKernelGGL((gemm_fast<BM, BN, WAVES_M, WAVES_N, EPI, BIAS, NA, NB, KALIGNED, kPingPong>),
+                     dim3(grid), dim3(64 * WAVES_M * WAVES_N), 0, st, p);
+}
+
+template <int BM, int BN, int WAVES_M, int WAVES_N, int EPI, bool BIAS, int NA = GEMM_RING_A,
+          int NB = GEMM_RING_B>
+void launch_fast_cfg(GemmArgs& p, hipStream_t st) {
+  if (p.k % 128 == 0) launch_tile<BM, BN, WAVES_M, WAVES_N, EPI, BIAS, NA, NB, true>(p, st);
+  else launch_tile<BM, BN, WAVES_M, WAVES_N, EPI, BIAS, NA, NB, false>(p, st);
+}
+
+// The tiles of 8 waves on a 2x4 grid: K % 128 == 0 only. With any other K
+// 256x128 and 128x256 run 4 waves of 128x64 / 64x128, and the rest, which have
+// no kernel for it, the 128x128 tile (the same outputs); the automatic choice
+// takes none of them there.
+template <int BM, int BN, int EPI, bool BIAS, int NA, int NB>
+void launch_mid_cfg(GemmArgs& p, hipStream_t st) {
+  constexpr bool kOwnRagged = BM * BN == 256 * 128 && (BM == 256 || BN == 256);
+  if (p.k % 128 == 0) launch_tile<BM, BN, 2, 4, EPI, BIAS, NA, NB, true>(p, st);
+  else if constexpr (kOwnRagged) launch_tile<BM, BN, 2, 2, EPI, BIAS, GEMM_RING_A, GEMM_RING_B, false>(p, st);
+  else launch_tile<128, 128, 2, 2, EPI, BIAS, GEMM_RING_A, GEMM_RING_B, false>(p, st);
 }
 
 // The persistent 256x256 block, streamed (K % 128 == 0 and K >= 256, else one
@@ -1365,13 +1375,13 @@ void launch_fast(int tile, GemmArgs& p, hipStream_t st) {
     // 8 waves of 64x96: 192-column tiles fill the CUs where 256-column ones leave a
     // partial wave (N = 5120 at M = 2048: 216 tiles instead of 160).
     case LR_TILE_256x192: launch_fast_cfg<256, 192, 4, 2, EPI, BIAS>(p, st); break;
-    case LR_TILE_256x128: launch_fast_cfg<256, 128, 2, 4, EPI, BIAS, 3, 2, false>(p, st); break;
-    case LR_TILE_128x256: launch_fast_cfg<128, 256, 2, 4, EPI, BIAS, 3, 2, false>(p, st); break;
-    case LR_TILE_224x256: launch_fast_cfg<224, 256, 2, 4, EPI, BIAS, 3, 2, false>(p, st); break;
-    case LR_TILE_160x256: launch_fast_cfg<160, 256, 2, 4, EPI, BIAS, 3, 2, false>(p, st); break;
-    case LR_TILE_192x128: launch_fast_cfg<192, 128, 2, 4, EPI, BIAS, 3, 3, false>(p, st); break;
-    case LR_TILE_128x192: launch_fast_cfg<128, 192, 2, 4, EPI, BIAS, 3, 3, false>(p, st); break;
-    case LR_TILE_96x128: launch_fast_cfg<96, 128, 2, 4, EPI, BIAS, 4, 4, false>(p, st); break;
+    case LR_TILE_256x128: launch_mid_cfg<256, 128, EPI, BIAS, 3, 2>(p, st); break;
+    case LR_TILE_128x256: launch_mid_cfg<128, 256, EPI, BIAS, 3, 2>(p, st); break;
+    case LR_TILE_224x256: launch_mid_cfg<224, 256, EPI, BIAS, 3, 2>(p, st); break;
+    case LR_TILE_160x256: launch_mid_cfg<160, 256, EPI, BIAS, 3, 2>(p, st); break;
+    case LR_TILE_192x128: launch_mid_cfg<192, 128, EPI, BIAS, 3, 3>(p, st); break;
+    case LR_TILE_128x192: launch_mid_cfg<128, 192, EPI, BIAS, 3, 3>(p, st); break;
+    case LR_TILE_96x128: launch_mid_cfg<96, 128, EPI, BIAS, 4, 4>(p, st); break;
     // 4 waves of 64x64; 80 KB of rings: 2 blocks per CU.
     case LR_TILE_128x128: launch_fast_cfg<128, 128, 2, 2, EPI, BIAS>(p, st); break;
     // 4 waves of 64x32 (24 KB k-steps), both operands GEMM_DEPTH_SMALL - 1

@@ -118,8 +118,16 @@ def _launch(a, b, row_scale, column_scale, bias, out, epilogue, tile, residual=N
 _CANDIDATES = (None, (256, 256), "persistent", (192, 256), (256, 192), (256, 128), (128, 256),
                (128, 128), (64, 128), (256, 80), (128, 160), (64, 80), (224, 256), (160, 256),
                (192, 128), (128, 192), (96, 128))
+# Tiles that exist for K % 128 == 0 only. With another K they run (128, 128),
+# "persistent" (256, 256).
+_ALIGNED_ONLY = frozenset({"persistent", (224, 256), (160, 256), (192, 128), (128, 192), (96, 128)})
 _selected: dict[tuple, object] = {}
 _prefixes: dict[int, tuple] = {}
+
+
+def _candidates(k):
+    """The candidates that run a kernel of their own at this K."""
+    return _CANDIDATES if k % 128 == 0 else tuple(t for t in _CANDIDATES if t not in _ALIGNED_ONLY)
 
 
 def _autotune_enabled() -> bool:
@@ -191,7 +199,7 @@ def _tuned_tile(a, b, row_scale, column_scale, bias, out, epilogue, residual, ta
     extra = dict(residual=residual, table=table, indices=indices, sequence=sequence,
                  gate_slot=gate_slot, splits=None)
     best, best_us = None, float("inf")
-    for candidate in _CANDIDATES:
+    for candidate in _candidates(k):
         try:
             _launch(*args, candidate if candidate is not None else "auto", **extra)
         except ValueError:

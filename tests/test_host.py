@@ -218,3 +218,13 @@ def test_int8_tma_entry_checks_layout():
         int8_tma.matmul(a, w.t().contiguous(), s, torch.ones(32))      # stride (32, 1), not (1, K)
     with pytest.raises(ValueError, match="TMA requires"):
         int8_tma.matmul(a.float(), w.t(), s, torch.ones(32))
+
+
+def test_autotune_candidates_run_their_own_kernel():
+    """With K off the k-step the tiles that have no kernel for it, and run
+    another tile's, are not timed under their own name."""
+    assert int8_gemm._candidates(384) == int8_gemm._CANDIDATES
+    ragged = int8_gemm._candidates(400)
+    assert ragged[0] is None and {(256, 128), (128, 256), (128, 128)} < set(ragged)
+    assert not int8_gemm._ALIGNED_ONLY & set(ragged)
+    assert int8_gemm._ALIGNED_ONLY < set(int8_gemm._CANDIDATES)

@@ -1493,52 +1493,83 @@ int tile_cols(int tile) { return tile_shape(tile).cols; }
 // idle CUs, and cost a second launch and the write and read of S int32 partial
 // outputs (9 TB/s: they stay in the 256 MB cache).
 //
-// Fitted (log least squares, 6% rms over 5600 points) to graph-replayed times
-// with rotating weights: 12 tiles, up to 8 slices, M = 1 to 16385 on the eight
-// projections of the Flash model and of the 5120-wide block, bf16 and gated
-// epilogues. Over those 320 shapes its choice is within 1.1% of the fastest
-// (geometric mean), and 9% faster than the rules before it, which knew
-// neither the tiles marked * nor splits below K = 16384. Examples, before ->
-// now: M = 32, N = 5376, K = 7168 20.7 -> 15.1 us (64x80 in 3 slices);
-// M = 256, N = 5376, K = 14336 54.6 -> 36.3 us (128x192* in 4); M = 878, same N, K
-// 104 -> 78 us (128x160); M = 1500, N = 5120, K = 5120 47 -> 41 us (128x256*);
-// M = 10240, N = 5120, K = 20480 886 -> 804 us (224x256*).
+// The constants were fitted (log least squares) to graph-replayed times with
+// rotating weights on the eight projections of the Flash model and of the
+// 5120-wide block (N * K from 26 to 154 million, K from 5120 to 20480), all but
+// the factor of 192x256, 0.96 in that fit: at 1.0 the 12288-token out-proj and
+// FFN-down take 256x256, as fast or faster in the projection chain. Below that
+// range weights, and soon both operands, stay in the caches, and the fixed
+// costs hide better the smaller the tile: `light`, 0 at the range's edge and
+// near 1 for the smallest weights, blends in a second factor per tile, cheaper
+// bytes and splits, and a smaller base, fitted to 3400 shapes with M from 1 to
+// 16384, N from 64 to 32768 and K from 128 to 24576.
 struct AutoTile {
   int id, rows, cols;
-  double factor;  // against the model: 64x128 and 128x160 run one wave per SIMD
+  double factor;  // against the model: 64x128, 128x160 and 128x128 run one wave per SIMD
+  double light;   // times this for light shapes
 };
 constexpr AutoTile kAutoTiles[] = {
-    {LR_TILE_256x256, 256, 256, 1.0},    {LR_TILE_224x256, 224, 256, 1.0},
-    {LR_TILE_192x256, 192, 256, 1.0},   {LR_TILE_160x256, 160, 256, 1.0},
-    {LR_TILE_256x128, 256, 128, 1.0},   {LR_TILE_128x256, 128, 256, 1.0},
-    {LR_TILE_192x128, 192, 128, 0.97},  {LR_TILE_128x192, 128, 192, 1.0},
-    {LR_TILE_128x160, 128, 160, 1.03},   {LR_TILE_96x128, 96, 128, 1.0},
-    {LR_TILE_64x128, 64, 128, 1.05},     {LR_TILE_64x80, 64, 80, 0.96},
+    {LR_TILE_256x256, 256, 256, 1.0, 1.225},  {LR_TILE_224x256, 224, 256, 1.0, 1.18},
+    {LR_TILE_192x256, 192, 256, 1.0, 1.14},   {LR_TILE_160x256, 160, 256, 1.0, 1.12},
+    {LR_TILE_256x128, 256, 128, 1.0, 1.145},  {LR_TILE_128x256, 128, 256, 1.0, 1.075},
+    {LR_TILE_192x128, 192, 128, 0.97, 1.18},  {LR_TILE_128x192, 128, 192, 1.0, 1.135},
+    {LR_TILE_128x160, 128, 160, 1.03, 1.085}, {LR_TILE_96x128, 96, 128, 1.0, 1.03},
+    {LR_TILE_64x128, 64, 128, 1.05, 0.875},   {LR_TILE_64x80, 64, 80, 0.96, 0.95},
 };
+// Tiles that only ragged_tile's rules take.
+constexpr AutoTile kRuleTiles[] = {{LR_TILE_256x192, 256, 192, 1.06, 1.175},
+                                   {LR_TILE_128x128, 128, 128, 1.3, 0.792}};
 // Automatic splits stay below this many slice bytes and slices: more never
 // measured faster by more than 7%, and callers hold the workspace.
 constexpr int64_t kAutoSliceBytes = 22LL << 20;
 constexpr int kAutoSlices = 8;
 
-double model_us(const AutoTile& t, int64_t m, int64_t n, int64_t k, int splits, int64_t cus) {
-  const int64_t tiles = ((m + t.rows - 1) / t.rows) * ((n + t.cols - 1) / t.cols) * splits;
-  const int64_t steps = ((k + 127) / 128 + splits - 1) / splits;
-  const int64_t full = tiles / cus, rest = tiles % cus;
-  const double waves = (double)full + (rest ? 0.9 + 0.1 * (double)rest / (double)cus : 0.0);
+// Whether the model was fitted on weights of this size and depth.
+bool fitted(int64_t n, int64_t k) {
+  const double weights = (double)n * (double)k;
+  return weights >= 26.2e6 && weights <= 154.2e6 && k >= 5120 && k <= 20480;
+}
+
+// What the model needs of a shape besides its tile.
+struct ModelShape {
+  int64_t m, n, k, cus;
+  double light, bytes, base, depth, weights;
+  ModelShape(int64_t m_, int64_t n_, int64_t k_, int64_t cus_) : m(m_), n(n_), k(k_), cus(cus_) {
+    weights = (double)n * (double)k * 1e-6;
+    const double size = weights < 26.2 ? weights / 26.2 : 1.0;
+    depth = k < 5120 ? (double)k / 5120 : 1.0;
+    light = 1.0 - size;
+    bytes = size < 1.0 ? std::fmax(0.52, std::pow(size, 0.285)) : 1.0;
+    base = 4.2 * (depth < 1.0 ? std::fmax(0.305, std::pow(depth, 0.47)) : 1.0);
+  }
+};
+
+double model_us(const AutoTile& t, const ModelShape& p, int splits) {
+  const int64_t tiles = ((p.m + t.rows - 1) / t.rows) * ((p.n + t.cols - 1) / t.cols) * splits;
+  const int64_t steps = ((p.k + 127) / 128 + splits - 1) / splits;
+  auto waves_of = [&](int64_t slots) {
+    const int64_t full = tiles / slots, rest = tiles % slots;
+    return (double)full + (rest ? 0.9 + 0.1 * (double)rest / (double)slots : 0.0);
+  };
+  double waves = waves_of(p.cus);
+  // Two blocks share a CU: the pair is done before twice the time of one.
+  if (tiles > p.cus && t.id == LR_TILE_64x80) waves *= 1.0 - 0.23 * p.light;
+  if (tiles > p.cus && t.id == LR_TILE_128x128) waves = 2.0 * waves_of(2 * p.cus) * (0.675 + 0.12 * p.depth);
   const double outputs = t.rows * t.cols * 1e-3;
-  const double bytes = 0.0624 + 0.00163 * (double)((m < t.rows ? m : t.rows) + t.cols);
+  const double bytes = (0.0624 + 0.00163 * (double)((p.m < t.rows ? p.m : t.rows) + t.cols)) * p.bytes;
   const double mfma = 0.01425 * outputs;
-  const double loop = waves * t.factor *
+  const double loop = waves * t.factor * (1.0 + p.light * (t.light - 1.0)) *
                       (2.7 + 0.054 * outputs + std::sqrt(bytes * bytes + mfma * mfma) * (double)steps);
-  const double weights = (double)n * (double)k * 1e-6 / 5.5;
-  double us = 4.2 + std::cbrt(loop * loop * loop + weights * weights * weights);
-  if (splits > 1) us += 2.6 + (double)splits * (double)m * (double)n * 8e-6 / 9.0;
+  const double weights = p.weights / 5.5;
+  double us = p.base + std::cbrt(loop * loop * loop + weights * weights * weights);
+  if (splits > 1) us += (2.6 + (double)splits * (double)p.m * (double)p.n * 8e-6 / 9.0) * (1.0 - 0.23 * p.light);
   return us;
 }
 
-// K % 128 != 0 (the mid-step loop of gemm_fast; the tiles of the model above
-// that exist for it lose up to 22% to these rules, which also take 128x128 and
-// 256x192): shape heuristic from measured sweeps (256 CUs, K = 5120 and 20480,
+// The rules for K % 128 != 0 (the mid-step loop of gemm_fast; the tiles of the
+// model above that exist for it lose up to 22% to these rules, which also take
+// 128x128 and 256x192), and a second opinion for the others (search, below): shape
+// heuristic from measured sweeps (256 CUs, K = 5120 and 20480,
 // M from 64 to 12288, N from 5120 to 20480). A launch takes as many
 // waves of tiles as its tile count fills the resident blocks of the device's
 // CUs (one 256x256, 192x256, 256x192 or 64x128 block per CU, two 128x128
@@ -1615,25 +1646,50 @@ int64_t split_workspace(int64_t m, int64_t n, int splits) { return splits > 1 ? 
 
 // Slices that fill one wave of the CUs with 128x160 tiles, at most 4, for a few
 // hundred rows at long K, where a split gains most (256 x 5120 x 20480: 36 us,
-// 42 unsplit); 1 elsewhere. Bounds what an automatic split may take for granted,
-// not its choice.
+// 42 unsplit); 1 elsewhere. The rules' split, and what a caller's workspace has
+// to hold there.
 int long_k_slices(int64_t m, int64_t n, int64_t k) {
   if (m <= 0 || n <= 0 || m > 256 || k < 16384 || k % 128 != 0 || n % 4 != 0) return 1;
   const int64_t s = compute_units() / (((m + 127) / 128) * ((n + 159) / 160));
   return s > 4 ? 4 : s > 1 ? (int)s : 1;
 }
 
-// The fastest (tile, splits) by the model, K % 128 == 0. splits 0: up to the workspace's
+// The fastest (tile, splits), K % 128 == 0. splits 0: up to the workspace's
 // bytes; else that many. `streamed`: the epilogue can take the persistent grid
 // where 256x256 tiles make two waves of the chip or more.
+//
+// The model decides, except where the rules of ragged_tile, with their splits of
+// long K, measured better than it prices them: 64x128 or 128x160 tiles that just
+// fill the CUs once (130-172 rows of N = 20480, K = 5120: 33 against 37 us), and, off
+// the fitted sizes, any tile that it puts within 3% of its own choice.
+//
+// Measured on 1400 shapes that no fit had seen (M from 1 to 16384, N from 64 to
+// 32768, K from 128 to 24576, half of them round sizes), geometric mean over the
+// fastest tile and split of each: 1.014; the rules alone 1.134, the projections'
+// constants everywhere 1.024. The last lost more than 4% to the rules on 101
+// shapes (up to 28%), mostly at K below 4096, where splits and large tiles cost
+// more than they save; this choice loses that much on 41 (up to 21%). On 300
+// shapes of the eight projections, M from 1 to 16384: 1.012, the rules 1.149, no
+// shape more than 4% slower. Examples, rules -> now: M = 32, N = 5376, K = 7168
+// 20.7 -> 15.1 us (64x80 in 3 slices); M = 256, N = 5376, K = 14336 54.6 -> 36.3 us
+// (128x192 in 4); M = 878, same N, K 104 -> 78 us (128x160); M = 1500, N = 5120,
+// K = 5120 47 -> 41 us (128x256).
 Plan search(int64_t m, int64_t n, int64_t k, int splits, int64_t workspace_bytes, bool streamed) {
   const int64_t cus = compute_units();
+  const ModelShape shape(m, n, k, cus);
   const int64_t steps = (k + 127) / 128;
   const int64_t budget = workspace_bytes < kAutoSliceBytes ? workspace_bytes : kAutoSliceBytes;
+  auto tiles_of = [&](const AutoTile& t) { return ((m + t.rows - 1) / t.rows) * ((n + t.cols - 1) / t.cols); };
+  auto price = [&](const AutoTile& t, int s) {
+    const double us = model_us(t, shape, s);
+    // The streamed grid against one tile per workgroup: 1-2% faster, 10% up to K = 1024.
+    return t.id == LR_TILE_256x256 && streamed && s == 1 && tiles_of(t) >= 2 * cus
+               ? us * (0.985 - 0.1 * (1.0 - shape.depth)) : us;
+  };
   Plan best{LR_TILE_256x256, splits > 0 ? splits : 1};
   double best_us = 0.0;
   for (const AutoTile& t : kAutoTiles) {
-    const int64_t tiles = ((m + t.rows - 1) / t.rows) * ((n + t.cols - 1) / t.cols);
+    const int64_t tiles = tiles_of(t);
     int last = splits > 0 ? splits : 1;
     if (splits == 0 && n % 4 == 0) {
       // Slices of at least 4 k-steps that make at most about one wave.
@@ -1642,17 +1698,26 @@ Plan search(int64_t m, int64_t n, int64_t k, int splits, int64_t workspace_bytes
         ++last;
     }
     for (int s = splits > 0 ? splits : 1; s <= last; ++s) {
-      double us = model_us(t, m, n, k, s, cus);
-      // The streamed grid is 1-2% faster than one tile per workgroup.
-      if (t.id == LR_TILE_256x256 && streamed && s == 1 && tiles >= 2 * cus) us *= 0.985;
+      const double us = price(t, s);
       if (best_us == 0.0 || us < best_us) best_us = us, best = Plan{t.id, s};
     }
   }
-  return best;
+  Plan rule{ragged_tile(m, n, k), splits > 0 ? splits : 1};
+  const int slices = splits == 0 ? long_k_slices(m, n, k) : 1;
+  if (slices > 1 && split_workspace(m, n, slices) <= budget) rule = Plan{LR_TILE_128x160, slices};
+  const AutoTile* t = nullptr;
+  for (const AutoTile& a : kAutoTiles) t = a.id == rule.tile ? &a : t;
+  for (const AutoTile& a : kRuleTiles) t = a.id == rule.tile ? &a : t;
+  double margin = 1.03;
+  if (fitted(n, k)) {
+    const bool one_wave = rule.splits == 1 && 10 * tiles_of(*t) >= 9 * cus && tiles_of(*t) <= cus;
+    margin = one_wave && (t->id == LR_TILE_64x128 || t->id == LR_TILE_128x160) ? 1.1 : 0.0;
+  }
+  return price(*t, rule.splits) < margin * best_us ? rule : best;
 }
 
-// The fast-path schedule. tile LR_TILE_AUTO: by the model above (K % 128 != 0: by
-// the rules of ragged_tile, unsplit), and where the model
+// The fast-path schedule. tile LR_TILE_AUTO: by the search above (K % 128 != 0: by
+// the rules of ragged_tile, unsplit), and where that
 // takes 256x256 tiles over at least two waves of the chip and the epilogue is
 // bf16 or GELU, the persistent grid with streamed tiles, 1-2% faster than one
 // tile per workgroup (QKV 12288x15360x5120: 660 against 672 us, FFN-up 894
@@ -1661,7 +1726,7 @@ Plan search(int64_t m, int64_t n, int64_t k, int splits, int64_t workspace_bytes
 // against 265 us), so the gated and raw epilogues keep one tile per workgroup.
 // workspace_bytes: what an automatic split may use.
 //
-// The search takes about 2 us, so each thread keeps its last results by shape
+// The search takes 3 to 8 us, so each thread keeps its last results by shape
 // (a function of the arguments and the device's CU count alone).
 Plan plan(int64_t m, int64_t n, int64_t k, int tile, int splits, int64_t workspace_bytes, int epilogue) {
   if (tile != LR_TILE_AUTO) return Plan{tile, splits > 0 ? splits : 1};

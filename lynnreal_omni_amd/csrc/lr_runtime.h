@@ -25,6 +25,11 @@ inline int check_launch(const char* where) {
 // Compute units of the current device (cached per device; 256 if the query fails).
 int compute_units();
 
+// Rows per launch of a kernel with a block per row, for callers with more of them:
+// a grid of 2^32 threads or more in one dimension runs without an error, but only
+// as many as its count modulo 2^32.
+constexpr int64_t kRowsPerLaunch = 1LL << 23;
+
 inline bool aligned(const void* p, uintptr_t bytes) { return ((uintptr_t)p % bytes) == 0; }
 
 inline hipStream_t as_stream(void* s) { return reinterpret_cast<hipStream_t>(s); }

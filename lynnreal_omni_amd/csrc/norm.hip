@@ -45,6 +45,7 @@ struct NormArgs {
   int64_t sequence, hidden, table_rows, table_width;
   int shift_slot, scale_slot, gate_slot;
   float eps;
+  int64_t first;  // the row of block 0 in the kernels with a block per row
 };
 
 // Loads chunk c (elements 8c .. 8c+7) of a bf16 row of length n; elements at
@@ -101,7 +102,7 @@ __device__ __forceinline__ void lds_barrier() {
 template <int CPT, bool VEC, bool RESID, bool QUANT>
 __global__ __launch_bounds__(kThreads) void rms_adaln_kernel(NormArgs p) {
   __shared__ float red[kThreads];
-  const int64_t row = blockIdx.x;
+  const int64_t row = p.first + blockIdx.x;
   const int64_t H = p.hidden;
   const int64_t chunks = (H + 7) / 8;
   const int64_t tr = clamp_index(p.indices[row % p.sequence], p.table_rows);
@@ -528,7 +529,7 @@ __global__ __launch_bounds__(kThreads) void rms_adaln_row(NormArgs p) {
   __shared__ float slots[kThreads];
   __shared__ float maxima[4];
   const int64_t H = p.hidden;
-  const int64_t row = blockIdx.x;
+  const int64_t row = p.first + blockIdx.x;
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
   const uint32_t off = 16u * threadIdx.x;
   auto load = [&](const uint16_t* src, uint4 (&v)[CPT]) {
@@ -626,14 +627,22 @@ __global__ __launch_bounds__(kThreads) void rms_adaln_row(NormArgs p) {
   }
 }
 
+// kernel(p) with a block per row, over at most kRowsPerLaunch rows at a time.
+void launch_rows(void (*kernel)(NormArgs), NormArgs p, int64_t rows, hipStream_t st) {
+  for (p.first = 0; p.first < rows; p.first += kRowsPerLaunch) {
+    const int64_t left = rows - p.first;
+    hipLaunchKernelGGL(kernel, dim3((unsigned)(left < kRowsPerLaunch ? left : kRowsPerLaunch)), dim3(kThreads), 0,
+                       st, p);
+  }
+}
+
 template <bool RESID, bool QUANT, bool NT>
 void launch_row(const NormArgs& p, int64_t rows, hipStream_t st) {
-  const dim3 grid((unsigned)rows), block(kThreads);
   const int64_t chunks = p.hidden / 8;
-  if (chunks <= 256) hipLaunchKernelGGL((rms_adaln_row<1, RESID, QUANT, NT>), grid, block, 0, st, p);
-  else if (chunks <= 512) hipLaunchKernelGGL((rms_adaln_row<2, RESID, QUANT, NT>), grid, block, 0, st, p);
-  else if (chunks <= 768) hipLaunchKernelGGL((rms_adaln_row<3, RESID, QUANT, NT>), grid, block, 0, st, p);
-  else hipLaunchKernelGGL((rms_adaln_row<4, RESID, QUANT, NT>), grid, block, 0, st, p);
+  if (chunks <= 256) launch_rows(rms_adaln_row<1, RESID, QUANT, NT>, p, rows, st);
+  else if (chunks <= 512) launch_rows(rms_adaln_row<2, RESID, QUANT, NT>, p, rows, st);
+  else if (chunks <= 768) launch_rows(rms_adaln_row<3, RESID, QUANT, NT>, p, rows, st);
+  else launch_rows(rms_adaln_row<4, RESID, QUANT, NT>, p, rows, st);
 }
 
 // Inputs of up to 24 MB are read through the caches, where the kernel that
@@ -716,9 +725,7 @@ int launch_norm(const NormArgs& p, int64_t rows, bool vec, hipStream_t st) {
   if (need > 16)
     return fail(LR_EUNSUPPORTED, "rms_adaln: hidden=%lld not supported (max %d)",
                 (long long)p.hidden, 16 * 8 * kThreads);
-#define LR_NORM_LAUNCH(C, V)                                                                  \
-  hipLaunchKernelGGL((rms_adaln_kernel<C, V, RESID, QUANT>), dim3((unsigned)rows), dim3(kThreads), \
-                     0, st, p)
+#define LR_NORM_LAUNCH(C, V) launch_rows(rms_adaln_kernel<C, V, RESID, QUANT>, p, rows, st)
   if (vec && need <= 8) LR_NORM_LAUNCH(8, true);
   else if (vec) LR_NORM_LAUNCH(16, true);
   else if (need <= 1) LR_NORM_LAUNCH(1, false);

@@ -197,19 +197,7 @@ __global__ __launch_bounds__(kThreads) void epilogue1(const int32_t* __restrict_
   out[e] = (uint16_t)(pack_bf2(v, 0.0f) & 0xffffu);
 }
 
-}  // namespace
-}  // namespace lr
-
-using namespace lr;
-
-extern "C" int lr_quantize_rows(const void* x, int64_t rows, int64_t width, int8_t* q,
-                                float* scales, void* stream) {
-  LR_REQUIRE(rows >= 0 && width >= 0, "quantize_rows: negative shape (%lld, %lld)",
-             (long long)rows, (long long)width);
-  if (rows == 0) return LR_OK;
-  LR_REQUIRE(x && q && scales, "quantize_rows: null pointer");
-  LR_REQUIRE(rows <= 0x7fffffffLL, "quantize_rows: too many rows (%lld)", (long long)rows);
-  hipStream_t st = as_stream(stream);
+int launch_quant(const void* x, int8_t* q, float* scales, int64_t rows, int64_t width, hipStream_t st) {
   const int64_t chunks = width / 8;
   const bool vec = width % 8 == 0 && aligned(x, 16) && aligned(q, 8) && chunks <= 16 * kThreads &&
                    width > 0;
@@ -231,6 +219,40 @@ extern "C" int lr_quantize_rows(const void* x, int64_t rows, int64_t width, int8
   return check_launch("quantize_rows");
 }
 
+template <typename T>
+int launch_quant_typed(const T* x, int8_t* q, float* scales, int64_t rows, int64_t width, hipStream_t st) {
+  hipLaunchKernelGGL(quantize_rows_typed<T>, dim3((unsigned)rows), dim3(kThreads), 0, st, x, q, scales, width);
+  return check_launch("quantize_rows");
+}
+
+// launch(x, q, scales, rows) over at most kRowsPerLaunch rows at a time.
+template <typename T, typename F>
+int in_slices(const T* x, int8_t* q, float* scales, int64_t rows, int64_t width, F launch) {
+  int rc = LR_OK;
+  for (int64_t r = 0; r < rows && rc == LR_OK; r += kRowsPerLaunch)
+    rc = launch(x + r * width, q + r * width, scales + r, rows - r < kRowsPerLaunch ? rows - r : kRowsPerLaunch);
+  return rc;
+}
+
+}  // namespace
+}  // namespace lr
+
+using namespace lr;
+
+extern "C" int lr_quantize_rows(const void* x, int64_t rows, int64_t width, int8_t* q,
+                                float* scales, void* stream) {
+  LR_REQUIRE(rows >= 0 && width >= 0, "quantize_rows: negative shape (%lld, %lld)",
+             (long long)rows, (long long)width);
+  if (rows == 0) return LR_OK;
+  LR_REQUIRE(x && q && scales, "quantize_rows: null pointer");
+  LR_REQUIRE(rows <= 0x7fffffffLL, "quantize_rows: too many rows (%lld)", (long long)rows);
+  hipStream_t st = as_stream(stream);
+  return in_slices(static_cast<const uint16_t*>(x), q, scales, rows, width,
+                   [&](const uint16_t* from, int8_t* to, float* scale, int64_t count) {
+                     return launch_quant(from, to, scale, count, width, st);
+                   });
+}
+
 extern "C" int lr_quantize_rows_typed(const void* x, int dtype, int64_t rows, int64_t width,
                                       int8_t* q, float* scales, void* stream) {
   LR_REQUIRE(dtype == LR_DTYPE_BF16 || dtype == LR_DTYPE_F16 || dtype == LR_DTYPE_F32,
@@ -242,13 +264,11 @@ extern "C" int lr_quantize_rows_typed(const void* x, int dtype, int64_t rows, in
   LR_REQUIRE(x && q && scales, "quantize_rows: null pointer");
   LR_REQUIRE(rows <= 0x7fffffffLL, "quantize_rows: too many rows (%lld)", (long long)rows);
   hipStream_t st = as_stream(stream);
-  if (dtype == LR_DTYPE_F16)
-    hipLaunchKernelGGL(quantize_rows_typed<_Float16>, dim3((unsigned)rows), dim3(kThreads), 0, st,
-                       (const _Float16*)x, q, scales, width);
-  else
-    hipLaunchKernelGGL(quantize_rows_typed<float>, dim3((unsigned)rows), dim3(kThreads), 0, st,
-                       (const float*)x, q, scales, width);
-  return check_launch("quantize_rows");
+  auto launch = [&](auto* from, int8_t* to, float* scale, int64_t count) {
+    return launch_quant_typed(from, to, scale, count, width, st);
+  };
+  if (dtype == LR_DTYPE_F16) return in_slices(static_cast<const _Float16*>(x), q, scales, rows, width, launch);
+  return in_slices(static_cast<const float*>(x), q, scales, rows, width, launch);
 }
 
 extern "C" int lr_int8_epilogue(const int32_t* acc, const float* a_scale, const float* w_scale,

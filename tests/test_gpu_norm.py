@@ -109,7 +109,7 @@ def test_quantizer_branch_for_huge_rows_one_table_row(kernel):
     """Rows whose modulated absmax is at or above 2^80 take the corrected
     quotient; the rest take the three-operation one. One table row whose scale
     slots are 2^86 makes every nonzero row huge, while all-zero input rows stay
-    at |y| = |shift|: both branches run in one launch of the one-row path."""
+    at |y| = |shift|: both branches run in one launch."""
     x, u, w, table, idx = case(1, 4096, 5120, 1, 21)
     table[:, 1 * 5120:2 * 5120] = BIG    # scale slot of (0, 1)
     table[:, 4 * 5120:5 * 5120] = BIG    # scale slot of (3, 4)
@@ -129,8 +129,9 @@ def test_quantizer_branch_for_huge_rows_one_table_row(kernel):
 @pytest.mark.parametrize("kernel", ["rms_adaln_quant", "residual_rms_quant"])
 def test_quantizer_branch_for_huge_rows_across_frame_runs(kernel):
     """The C5 per-frame layout with the scale slots of frames 1, 3 and 5 set to
-    2^86: slices that span a frame boundary (two runs of table rows) switch
-    between the two quotient forms inside one slice."""
+    2^86. Without a residual, slices that span a frame boundary (two runs of table
+    rows) switch between the two quotient forms inside one slice; rows of 5120 with
+    one have a block each (test_gpu_norm_stream.py has the residual slices)."""
     x, u, w, table, idx = case(1, 12605, 5120, 6, 22, True)
     for frame in (1, 3, 5):
         table[frame, 1 * 5120:2 * 5120] = BIG

@@ -2,9 +2,9 @@
 oracle: the quantizer (model/int8.py:66-67), the fused norm + modulate (+ quant)
 and residual variants (model/kernels.py:48-128, :405-419) and the gated residual
 (:131-153). Widths cover the register-resident kernels (multiples of 8 up to
-8192), the one-row-per-block kernels and element-wise tails; row counts cover
-partial persistent slices; tables have one to six rows with random indices.
-All outputs bit-exact."""
+8192) and the kernels with element-wise tails; up to 900 rows, for which the norms
+run a block per row (test_gpu_norm_stream.py has the persistent grid's cases);
+tables have one to six rows with random indices. All outputs bit-exact."""
 import numpy as np
 import pytest
 import torch

@@ -8,6 +8,7 @@ is smaller, then refused beyond the array's size.
 import pytest
 import torch
 
+from graph_nodes import kernels
 from lynnreal_omni_amd import _lib
 
 pytestmark = pytest.mark.gpu
@@ -84,28 +85,26 @@ def test_noalloc_forced_split_and_limit():
     assert not out.any()
 
 
-def test_automatic_choice_takes_the_scratch_only_at_long_k():
-    """Calls whose automatic split is new with the workspace entry point (few
-    rows at short K, wide N at long K) leave the shared array alone: overlapping
-    noalloc calls stay independent there. The outputs are the same."""
+@pytest.mark.parametrize("m,n,k,launches", [(32, 5376, 7168, 1), (32, 1024, 4096, 1), (256, 5120, 20480, 2)])
+def test_automatic_choice_takes_the_scratch_only_at_long_k(m, n, k, launches):
+    """All three shapes are split where a workspace is given. Without one, the
+    shared array is taken at long K only (a second kernel sums its slices), so that
+    overlapping calls of the others stay independent. The outputs are the same."""
     lib = _lib.load()
-    streams = [torch.cuda.Stream() for _ in range(2)]
-    for m, n, k in ((32, 5376, 7168), (200, 20480, 16384)):
-        sets = [_inputs(m, n, k, seed) for seed in (5, 6)]
-        want = []
-        for a, w, rs, cs, bias in sets:
-            out = torch.empty(m, n, dtype=torch.bfloat16, device="cuda")
-            assert lib.lr_int8_gemm(*_args(a, w, rs, cs, bias, out, _lib.EPI_BF16), _lib.TILE_AUTO,
-                                    torch.cuda.current_stream().cuda_stream) == _lib.LR_OK
-            want.append(out)
-        got = [torch.empty_like(o) for o in want]
-        torch.cuda.synchronize()
-        for _ in range(8):
-            for (a, w, rs, cs, bias), out, st in zip(sets, got, streams):
-                assert lib.lr_int8_gemm_noalloc(*_args(a, w, rs, cs, bias, out, _lib.EPI_BF16), 0,
-                                                _lib.TILE_AUTO, st.cuda_stream) == _lib.LR_OK
-        torch.cuda.synchronize()
-        assert all(torch.equal(g, o) for g, o in zip(got, want)), (m, n, k)
+    assert lib.lr_int8_gemm_workspace_size(m, n, k, 0, _lib.TILE_AUTO) > 0
+    a, w, rs, cs, bias = _inputs(m, n, k, 5)
+    want, got = (torch.empty(m, n, dtype=torch.bfloat16, device="cuda") for _ in range(2))
+    assert lib.lr_int8_gemm(*_args(a, w, rs, cs, bias, want, _lib.EPI_BF16), _lib.TILE_AUTO,
+                            torch.cuda.current_stream().cuda_stream) == _lib.LR_OK
+
+    def call():
+        assert lib.lr_int8_gemm_noalloc(*_args(a, w, rs, cs, bias, got, _lib.EPI_BF16), 0, _lib.TILE_AUTO,
+                                        torch.cuda.current_stream().cuda_stream) == _lib.LR_OK
+
+    call()
+    torch.cuda.synchronize()
+    assert torch.equal(got, want)
+    assert len(kernels(call)) == launches
 
 
 def test_long_k_workspace_below_its_slices_is_refused():

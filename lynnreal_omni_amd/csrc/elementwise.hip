@@ -250,7 +250,7 @@ __global__ __launch_bounds__(kThreads) void gelu_quant_any(const uint16_t* __res
 
 int blocks_for(int64_t work, unsigned* out) {
   const int64_t b = (work + kThreads - 1) / kThreads;
-  if (b > 0x7fffffffLL) return fail(LR_EUNSUPPORTED, "elementwise: problem too large (not supported)");
+  if (b > kMaxBlocks) return fail(LR_EUNSUPPORTED, "elementwise: problem too large (not supported)");
   *out = (unsigned)b;
   return LR_OK;
 }
@@ -307,7 +307,7 @@ extern "C" int lr_swiglu_quant(const void* p, int8_t* q, float* scales, int64_t 
   LR_REQUIRE(rows >= 0 && inner > 0, "swiglu_quant: bad shape");
   if (rows == 0) return LR_OK;
   LR_REQUIRE(p && q && scales, "swiglu_quant: null pointer");
-  LR_REQUIRE(rows <= 0x7fffffffLL, "swiglu_quant: too many rows");
+  LR_REQUIRE(rows <= kMaxBlocks, "swiglu_quant: too many rows");
   hipStream_t st = as_stream(stream);
   const int64_t cpr = inner / 8;
   const bool vec = inner % 8 == 0 && aligned(p, 16) && aligned(q, 8) && cpr <= 16 * kThreads;
@@ -348,7 +348,7 @@ extern "C" int lr_gelu_quant(const void* x, int8_t* q, float* scales, int64_t ro
   LR_REQUIRE(rows >= 0 && width > 0, "gelu_quant: bad shape");
   if (rows == 0) return LR_OK;
   LR_REQUIRE(x && q && scales, "gelu_quant: null pointer");
-  LR_REQUIRE(rows <= 0x7fffffffLL, "gelu_quant: too many rows");
+  LR_REQUIRE(rows <= kMaxBlocks, "gelu_quant: too many rows");
   hipStream_t st = as_stream(stream);
   const int64_t chunks = width / 8;
   const bool vec = width % 8 == 0 && aligned(x, 16) && aligned(q, 8) && chunks <= 16 * kThreads;

@@ -244,8 +244,8 @@ extern "C" int lr_gather_rows(const void* src, const int64_t* index, void* dst, 
   LR_REQUIRE(src && index && dst, "gather_rows: null pointer");
   hipStream_t st = as_stream(stream);
   if (row_bytes % 16 == 0 && aligned(src, 16) && aligned(dst, 16)) {
-    LR_REQUIRE(rows <= 0x7fffffffLL, "gather_rows: too many rows");
     const int64_t units = row_bytes / 16;
+    LR_REQUIRE(rows <= kMaxBlocks || (units < 64 && rows * units < 0x7fffff00LL), "gather_rows: too many rows");
     const uint4* from = static_cast<const uint4*>(src);
     uint4* to = static_cast<uint4*>(dst);
     const dim3 grid((unsigned)rows), block(kThreads);
@@ -267,7 +267,7 @@ extern "C" int lr_gather_rows(const void* src, const int64_t* index, void* dst, 
   } else {
     const int64_t total = rows * row_bytes;
     const int64_t blocks = (total + kThreads - 1) / kThreads;
-    LR_REQUIRE(blocks <= 0x7fffffffLL, "gather_rows: too many bytes");
+    LR_REQUIRE(blocks <= kMaxBlocks, "gather_rows: too many bytes");
     hipLaunchKernelGGL(gather_rows_bytes, dim3((unsigned)blocks), dim3(kThreads), 0, st,
                        (const uint8_t*)src, index, (uint8_t*)dst, src_rows, dst_rows, row_bytes,
                        total);
@@ -288,7 +288,7 @@ extern "C" int lr_flash_restore(const void* full, const void* current, const voi
   if (width % 8 == 0 && aligned(full, 16) && aligned(current, 16) && aligned(input, 16) &&
       aligned(out, 16)) {
     const int64_t blocks = 8 * ((out_rows + 7) / 8);  // a whole number of rows per XCD
-    LR_REQUIRE(blocks <= 0x7fffffffLL, "flash_restore: too many rows");
+    LR_REQUIRE(blocks <= kMaxBlocks, "flash_restore: too many rows");
     const int64_t units = width / 8;
 #define LR_RESTORE(C)                                                                              \
   hipLaunchKernelGGL(restore_rows8<C>, dim3((unsigned)blocks), dim3(kThreads), 0, st,               \
@@ -304,7 +304,7 @@ extern "C" int lr_flash_restore(const void* full, const void* current, const voi
   } else {
     const int64_t total = out_rows * width;
     const int64_t blocks = (total + kThreads - 1) / kThreads;
-    LR_REQUIRE(blocks <= 0x7fffffffLL, "flash_restore: too many elements");
+    LR_REQUIRE(blocks <= kMaxBlocks, "flash_restore: too many elements");
     hipLaunchKernelGGL(restore_rows_any, dim3((unsigned)blocks), dim3(kThreads), 0, st,
                        (const uint16_t*)full, (const uint16_t*)current, (const uint16_t*)input,
                        inverse, (uint16_t*)out, rows, compressed_rows, width, total, gain);
@@ -321,7 +321,7 @@ extern "C" int lr_flash_nearest_anchor(const float* positions, int64_t tokens,
   LR_REQUIRE(n_anchors > 0 && tokens > 0, "nearest_anchor: dropped rows but no anchors");
   LR_REQUIRE(positions && dropped && anchors && inverse, "nearest_anchor: null pointer");
   const int64_t blocks = (n_dropped + kAnchorRows - 1) / kAnchorRows;
-  LR_REQUIRE(blocks <= 0x7fffffffLL, "nearest_anchor: too many rows");
+  LR_REQUIRE(blocks <= kMaxBlocks, "nearest_anchor: too many rows");
   hipLaunchKernelGGL(nearest_anchor, dim3((unsigned)blocks), dim3(kThreads), 0, as_stream(stream),
                      positions, dropped, anchors, inverse, tokens, n_dropped, n_anchors);
   return check_launch("nearest_anchor");

@@ -25,9 +25,10 @@ inline int check_launch(const char* where) {
 // Compute units of the current device (cached per device; 256 if the query fails).
 int compute_units();
 
-// Rows per launch of a kernel with a block per row, for callers with more of them:
-// a grid of 2^32 threads or more in one dimension runs without an error, but only
-// as many as its count modulo 2^32.
+// Blocks of 256 threads that one launch may have: a grid of 2^32 threads or more in
+// one dimension runs without an error, but only as many as its count modulo 2^32.
+constexpr int64_t kMaxBlocks = (1LL << 24) - 1;
+// Rows per launch of a kernel with a block per row, for callers with more of them.
 constexpr int64_t kRowsPerLaunch = 1LL << 23;
 
 inline bool aligned(const void* p, uintptr_t bytes) { return ((uintptr_t)p % bytes) == 0; }

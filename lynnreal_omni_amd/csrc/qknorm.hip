@@ -254,7 +254,7 @@ extern "C" int lr_qk_norm_rope(const void* q, const void* k, const void* q_weigh
                           (rotary_dim == 0 || (aligned(cos, 16) && aligned(sin, 16)));
   if (!aligned_ok)
     return fail(LR_EUNSUPPORTED, "qk_norm_rope: rows must be 16-byte aligned");
-  LR_REQUIRE((batch * sequence + 3) / 4 < 0x7fffffffLL, "qk_norm_rope: too many tokens");
+  LR_REQUIRE((batch * sequence + 3) / 4 <= kMaxBlocks, "qk_norm_rope: too many tokens");
   // Per-token descriptors: a token's heads must span less than 2^31 bytes.
   LR_REQUIRE(heads * (q_head_stride > k_head_stride ? q_head_stride : k_head_stride) <
                  (1LL << 30) - 64 * head_dim,

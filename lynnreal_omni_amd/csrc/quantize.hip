@@ -283,7 +283,7 @@ extern "C" int lr_int8_epilogue(const int32_t* acc, const float* a_scale, const 
   if (vec) {
     const int64_t groups = m * (n / 4);
     const int64_t blocks = (groups + kThreads - 1) / kThreads;
-    LR_REQUIRE(blocks <= 0x7fffffffLL, "int8_epilogue: too large");
+    LR_REQUIRE(blocks <= kMaxBlocks, "int8_epilogue: too large");
     if (bias)
       hipLaunchKernelGGL(epilogue4<true>, dim3((unsigned)blocks), dim3(kThreads), 0, st,
                          (const int4*)acc, a_scale, w_scale, (const uint16_t*)bias, (uint2*)out,
@@ -295,7 +295,7 @@ extern "C" int lr_int8_epilogue(const int32_t* acc, const float* a_scale, const 
   } else {
     const int64_t total = m * n;
     const int64_t blocks = (total + kThreads - 1) / kThreads;
-    LR_REQUIRE(blocks <= 0x7fffffffLL, "int8_epilogue: too large");
+    LR_REQUIRE(blocks <= kMaxBlocks, "int8_epilogue: too large");
     hipLaunchKernelGGL(epilogue1, dim3((unsigned)blocks), dim3(kThreads), 0, st, acc, a_scale,
                        w_scale, (const uint16_t*)bias, (uint16_t*)out, total, n);
   }

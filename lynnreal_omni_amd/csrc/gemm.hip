@@ -1407,9 +1407,11 @@ void launch_fast(int tile, GemmArgs& p, hipStream_t st) {
     case LR_TILE_128x160: launch_fast_cfg<128, 160, 2, 2, EPI, BIAS, GEMM_SKINNY128_NA, GEMM_SKINNY128_NB>(p, st); break;
     // 8 waves of 96x64 (the 2x4 grid, so the early W refill): where 256x256
     // tiles leave the last wave a quarter empty (M = 12288, N = 5120: 960
-    // tiles = 3.75 waves) its 1280 tiles make 5 full waves. Each tile carries
-    // more fixed cost per op, so it pays only at long K: FFN-down (K = 20480)
-    // 865 against 881 us, out-proj (K = 5120) 231 against 224 us.
+    // tiles = 3.75 waves) its 1280 tiles make 5 full waves, at more fixed cost
+    // per op. Launched back to back that pays at long K (FFN-down, K = 20480, 865
+    // against 881 us; out-proj, K = 5120, 231 against 224 us). In the projection
+    // chain it does not (a step of 2910 us, 2921 with FFN-down and 2920 with
+    // out-proj on 192x256, 2929 with both), and the model leaves both to 256x256.
     case LR_TILE_192x256: launch_fast_cfg<192, 256, 2, 4, EPI, BIAS>(p, st); break;
     default: launch_fast_cfg<64, 128, 1, 4, EPI, BIAS, GEMM_DEPTH_SMALL, GEMM_DEPTH_SMALL>(p, st); break;
   }
@@ -1497,7 +1499,7 @@ int tile_cols(int tile) { return tile_shape(tile).cols; }
 // rotating weights on the eight projections of the Flash model and of the
 // 5120-wide block (N * K from 26 to 154 million, K from 5120 to 20480), all but
 // the factor of 192x256, 0.96 in that fit: at 1.0 the 12288-token out-proj and
-// FFN-down take 256x256, as fast or faster in the projection chain. Below that
+// FFN-down take 256x256, 10 and 12 us faster in the projection chain. Below that
 // range weights, and soon both operands, stay in the caches, and the fixed
 // costs hide better the smaller the tile: `light`, 0 at the range's edge and
 // near 1 for the smallest weights, blends in a second factor per tile, cheaper

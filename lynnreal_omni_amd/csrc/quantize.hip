@@ -5,8 +5,9 @@
 // kernel model/kernels.py:8-16 computes the same values). Narrow rows (under
 // 4096): one wave per row, four rows per 256-thread block; lane l holds 16-byte
 // chunks l, l+64, ... in registers, the absmax is a wave butterfly, and the
-// row is quantized from registers and written with 8-byte stores. Wider or few
-// rows: one 256-thread block per row, same scheme with a block reduction. HBM
+// row is quantized from registers and written with 8-byte stores. Rows of 4096 and
+// more, and at most 512 rows wider than 2048: one 256-thread block per row, same
+// scheme with a block reduction. HBM
 // traffic is the algorithmic 3 bytes/element plus 4 bytes/row.
 #include "lr_device.h"
 #include "lr_runtime.h"
@@ -43,12 +44,13 @@ __global__ __launch_bounds__(kThreads) void quantize_rows_wave(const uint4* __re
   if (lane == 0) scales[row] = s;
 }
 
-// One block per row, for rows of 4096 and more and for few rows of any width,
+// One block per row, for rows of 4096 and more and for few rows wider than 2048,
 // where a wave per row has more serial work than it hides. Loads and stores go
 // through descriptors that end with the row. NT: non-temporal loads, for inputs
 // past 32 MB; smaller ones are still in the caches from the kernel that wrote
-// them. Rows past 8192 are stored write-back (20480 wide, 12605 rows 116.7
-// against 123.9 us non-temporal), narrower ones non-temporally.
+// them. Rows past 8192 always load non-temporally (the other form is not built
+// for them) and are stored write-back (20480 wide, 12605 rows 116.7 against
+// 123.9 us non-temporal), narrower ones non-temporally.
 template <int CPT, bool NT>
 __global__ __launch_bounds__(kThreads) void quantize_rows_block(const uint4* __restrict__ x,
                                                                 uint2* __restrict__ q,

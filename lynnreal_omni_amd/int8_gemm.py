@@ -336,7 +336,10 @@ def linear_rows(rows, b, column_scale, bias):
         quantized, scale = quantize_rows(rows)
         return int8_matmul(quantized, b, scale, column_scale, bias)
     _lib.check_device(rows)
-    _lib.same_device(rows, b=b, column_scale=column_scale, bias=bias)
+    index = rows.get_device()
+    if (b.get_device() != index or column_scale.get_device() != index
+            or bias is not None and bias.get_device() != index):
+        _lib.same_device(rows, b=b, column_scale=column_scale, bias=bias)     # raises, naming the tensor
     slices = _workspace_bytes(m, n, k, 0, _lib.TILE_AUTO)
     scale_at = -(-m * k // 256) * 256
     slices_at = scale_at + -(-4 * m // 256) * 256

@@ -103,3 +103,20 @@ def test_tensors_of_the_fused_call(monkeypatch, name):
     setattr(layer, name, value)
     layer(X)
     assert all(a is b for a, b in zip(got[0], (layer.weight_int8, layer.weight_scale, layer.bias)))
+
+
+@pytest.mark.parametrize("where", ["instance", "subclass"])
+@pytest.mark.parametrize("name", ["weight_int8", "weight_scale", "bias"])
+def test_tensors_that_hide_a_buffer(monkeypatch, name, where):
+    """An attribute that hides the buffer of its name is what the fused call reads."""
+    got = []
+    monkeypatch.setattr(int8_gemm, "linear_rows", lambda rows, *tensors: got.append(tensors) or rows[:, :24])
+    layer = _layer()
+    other = getattr(layer, name).clone()
+    if where == "instance":
+        layer.__dict__[name] = other
+    else:      # as torch.nn.utils.parametrize does it
+        layer.__class__ = type("Own", (Int8Linear,), {name: property(lambda self: other)})
+    layer(X)
+    assert got[0][("weight_int8", "weight_scale", "bias").index(name)] is not layer._buffers[name]
+    assert all(a is b for a, b in zip(got[0], (layer.weight_int8, layer.weight_scale, layer.bias)))

@@ -274,7 +274,7 @@ __device__ __forceinline__ void norm_row(const NormArgs& p, int64_t row, const u
 #pragma unroll
       for (int e = 0; e < 8; ++e) xf[e] = xf[e] + round_bf(g[e] * uf[e]);
       r.x[m] = pack8(xf);
-      buf_store16(orow, 16u * lane, 1024u * m, r.x[m]);
+      buf_store16(orow, 16u * lane + 1024u * m, 0, r.x[m]);
       __builtin_amdgcn_sched_barrier(0);
     }
   }
@@ -327,7 +327,7 @@ __device__ __forceinline__ void norm_row(const NormArgs& p, int64_t row, const u
       amax = fmaxf(amax, __builtin_fabsf(xf[e]));
     }
     r.x[m] = pack8(xf);
-    if (!QUANT) buf_store16(orow, 16u * lane, 1024u * m, r.x[m]);
+    if (!QUANT) buf_store16(orow, 16u * lane + 1024u * m, 0, r.x[m]);
     __builtin_amdgcn_sched_barrier(0);
   }
   if (QUANT) {
@@ -388,7 +388,7 @@ __device__ __forceinline__ void norm_row_f32(const NormArgs& p, int64_t row, con
       f[m][e] = round_bf(t + sh[e]);
       amax = fmaxf(amax, __builtin_fabsf(f[m][e]));
     }
-    if (!QUANT) buf_store16(orow, 16u * lane, 1024u * m, pack8(f[m]));
+    if (!QUANT && CPL > 10) buf_store16(orow, 16u * lane + 1024u * m, 0, pack8(f[m]));
     __builtin_amdgcn_sched_barrier(0);
   }
   if (QUANT) {
@@ -412,6 +412,15 @@ __device__ __forceinline__ void norm_row_f32(const NormArgs& p, int64_t row, con
       }
     }
     if (lane == 0) p.scales[row] = s;
+  } else if (CPL <= 10) {
+    // All stores after the last chunk: 2 to 7% faster than one behind each chunk
+    // (1600 x 4096 8.1 us, 8.6; 12605 x 1024 with 6 table rows 13.8, 16.0), where the
+    // registers hold the row that long.
+#pragma unroll
+    for (int m = 0; m < CPL; ++m) {
+      buf_store16(orow, 16u * lane + 1024u * m, 0, pack8(f[m]));
+      if (CPL > 8) __builtin_amdgcn_sched_barrier(0);
+    }
   }
 }
 
@@ -656,8 +665,8 @@ void launch_row(const NormArgs& p, int64_t rows, hipStream_t st) {
   else launch_rows(rms_adaln_row<4, RESID, QUANT, NT>, p, rows, st);
 }
 
-// Inputs of up to 24 MB are read through the caches, where the kernel that
-// produced them left them (residual norm of 878 x 5376 9.4 against 10.8 us
+// Inputs of up to 24 MB are read through the caches, which keeps them there for
+// another pass over them (residual norm of 878 x 5376 9.4 against 10.8 us
 // non-temporal); larger ones non-temporally (12605 rows 85.3 against 91.6 us).
 template <bool RESID, bool QUANT>
 void launch_norm_row(const NormArgs& p, int64_t rows, hipStream_t st) {
@@ -710,25 +719,34 @@ bool launch_norm_stream(const NormArgs& p, int64_t rows, hipStream_t st) {
 
 // One row per block, or a persistent grid that stages its parameters once: the
 // staging (and, with several table rows, the search for their boundaries) costs
-// 3-6 us, which many rows repay and few do not. us, graph-replayed, one row per
-// block / streamed: norm + quant of 878 x 5376, 6 table rows 7.3 / 11.7, 3683
-// rows 17.6 / 19.3, 6144 rows 26.7 / 24.3, 12605 rows 51.6 / 47.3; one table row
-// 878 rows 7.0 / 7.5, 2048 rows 11.4 / 10.2; narrow rows cross earlier (1024 wide,
-// 6 table rows: 4096 rows 9.6 / 9.6). With a residual the row kernel has 5 blocks
-// per CU in flight where the streamed one has 8 waves of two rows each, and is
-// ahead at every count from 3072 columns on (12605 x 5120 82.5 / 87.4, 512 x 5120
-// 6.8 / 14.8); below, up to the counts here (2048 wide: 6144 rows 19.8 / 21.5).
-bool prefer_row_kernel(bool resid, int64_t rows, int64_t hidden, int64_t table_rows) {
-  if (resid) return hidden > 3072 || rows < (hidden >= 2048 ? 8192 : 3072);
-  if (table_rows == 1) return rows < (hidden > 3072 ? 1536 : 1024);
-  return rows < (hidden > 1024 ? 4096 : 2560);
+// 3-6 us, which many rows repay and few do not. us, graph-replayed over rotating
+// inputs, one row per block / streamed: norm + quant of 878 x 5376, 6 table rows 7.3
+// / 11.7, 3683 rows 17.6 / 19.3, 6144 rows 26.7 / 24.3, 12605 rows 51.6 / 47.3; one
+// table row 878 rows 7.0 / 7.5, 2048 rows 11.4 / 10.2; narrow rows cross earlier
+// (1024 wide, 6 table rows: 4096 rows 9.6 / 9.6). Without quantization the streamed
+// kernel has less to do: 878 x 5120 with one table row 7.5 / 6.8.
+// With a residual the row kernel has 5 blocks per CU in flight where the streamed one
+// has 8 waves of two rows each, and is ahead at every count from 3072 columns on
+// (12605 x 5120 85.6 / 95.9, 24576 rows 167 / 188, 512 rows 6.8 / 14.8; a loop over
+// the same 24576 rows, which then come from the caches, 164 / 150); below, up to the
+// counts here (2048 wide: 6144 rows 19.8 / 21.5), which narrow rows with one table
+// row reach first (512 wide: 1200 rows 5.1 / 4.0, 2600 rows 8.3 / 5.8).
+bool prefer_row_kernel(bool resid, bool quant, int64_t rows, int64_t hidden, int64_t table_rows) {
+  if (resid) {
+    if (hidden > 3072) return true;
+    if (hidden >= 1536) return rows < (hidden >= 2048 ? 8192 : 3072);
+    return rows < (table_rows == 1 ? 1024 : hidden > 768 ? 3072 : 2048);
+  }
+  if (table_rows > 1) return rows < (hidden > 1024 ? 4096 : 2560);
+  if (!quant && hidden > 3072 && hidden <= 5120) return rows < 768;
+  return rows < (hidden > 3072 ? 1536 : 1024);
 }
 
 template <bool RESID, bool QUANT>
 int launch_norm(const NormArgs& p, int64_t rows, bool vec, hipStream_t st) {
   const int64_t chunks = (p.hidden + 7) / 8;
   if (vec && chunks <= 1024) {
-    if (prefer_row_kernel(RESID, rows, p.hidden, p.table_rows) || !launch_norm_stream<RESID, QUANT>(p, rows, st))
+    if (prefer_row_kernel(RESID, QUANT, rows, p.hidden, p.table_rows) || !launch_norm_stream<RESID, QUANT>(p, rows, st))
       launch_norm_row<RESID, QUANT>(p, rows, st);
     return check_launch("rms_adaln");
   }

@@ -47,10 +47,13 @@ __global__ __launch_bounds__(kThreads) void quantize_rows_wave(const uint4* __re
 // One block per row, for rows of 4096 and more and for few rows wider than 2048,
 // where a wave per row has more serial work than it hides. Loads and stores go
 // through descriptors that end with the row. NT: non-temporal loads, for inputs
-// past 32 MB; smaller ones are still in the caches from the kernel that wrote
-// them. Rows past 8192 always load non-temporally (the other form is not built
-// for them) and are stored write-back (20480 wide, 12605 rows 116.7 against
-// 123.9 us non-temporal), narrower ones non-temporally.
+// past 32 MB; smaller ones are read through the caches, for layers that are called
+// on the same rows again (layer calls of 2048 x 5120 rows 51.6 us, 52.8
+// non-temporal); rows read once are faster non-temporally (2048 x 5120 from memory
+// 7.4 us, 8.1 through the caches; just written 5.5 and 6.1). Rows past 8192 always
+// load non-temporally (the other form is not built for them) and are stored
+// write-back (20480 wide, 12605 rows 116.7 against 123.9 us non-temporal), narrower
+// ones non-temporally.
 template <int CPT, bool NT>
 __global__ __launch_bounds__(kThreads) void quantize_rows_block(const uint4* __restrict__ x,
                                                                 uint2* __restrict__ q,
